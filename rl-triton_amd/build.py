@@ -21,6 +21,8 @@ import glob
 import os
 import subprocess
 import sys
+import tempfile
+from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 REPO = os.path.dirname(HERE)
@@ -72,7 +74,14 @@ def build_lib(force: bool = True, verbose: bool = False) -> str:
         return LIB
     hipcc = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
     tmp = LIB + ".tmp"
-    _run([hipcc, *FLAGS, f"-I{INCLUDE}", f"-I{CSRC}", *sources(), "-o", tmp], verbose)
+    with tempfile.TemporaryDirectory() as d:
+        # one translation unit per estimator, compiled side by side
+        objs = [os.path.join(d, os.path.basename(s) + ".o") for s in sources()]
+        compile_flags = [f for f in FLAGS if f != "-shared"]
+        with ThreadPoolExecutor(max_workers=min(len(objs), os.cpu_count() or 1)) as pool:
+            list(pool.map(lambda so: _run([hipcc, *compile_flags, f"-I{INCLUDE}", f"-I{CSRC}", "-c",
+                                           so[0], "-o", so[1]], verbose), zip(sources(), objs)))
+        _run([hipcc, "-fPIC", "-shared", f"--offload-arch={ARCH}", *objs, "-o", tmp], verbose)
     os.replace(tmp, LIB)
     return LIB
 

@@ -385,7 +385,7 @@ __device__ __forceinline__ void store_seg(E* __restrict__ p, int t0, int T, cons
 // Global (not __constant__) memory, so that selecting between it and a global operand keeps
 // a global load (a flat load would also count against the LDS counter).  All-zero bits are
 // also a bfloat16 zero.
-__device__ float g_zero[4] = {0.f, 0.f, 0.f, 0.f};
+static __device__ float g_zero[4] = {0.f, 0.f, 0.f, 0.f};
 template <class E>
 __device__ __forceinline__ const E* zero_src() { return reinterpret_cast<const E*>(g_zero); }
 
