@@ -20,7 +20,8 @@
 //
 // An estimator ("Op") supplies:
 //   Regs                      per-thread registers for S steps
-//   load(row, t0, T, R)       issue the segment's loads, clamped into the row
+//   load(at, R)               issue the segment's loads, clamped into the row (at: where the
+//                             segment lies, RowAt)
 //   prepare(R, row, t0, T)    everything derived from the loaded values (exp, ratios,
 //                             bootstrap selection)
 //   Halo / export / halo_load the one-step neighbour data the producer needs (values[t+1]
@@ -28,7 +29,7 @@
 //                             and read from global memory at wave/tile edges
 //   coef(...)                 per-step (add, mul) with truncation/bootstrap folded in;
 //                             padding steps (t >= T) are the identity map
-//   row_carry_src(row, T)     address of x[T] (backward) or x[-1] (forward), or nullptr (0)
+//   row_carry_src(at)         address of x[T] (backward) or x[-1] (forward), or nullptr (0)
 //   emit(...)                 outputs from the scanned x (and x one step further)
 #pragma once
 #include <hip/hip_runtime.h>
@@ -393,11 +394,52 @@ __device__ __forceinline__ const E* zero_src() { return reinterpret_cast<const E
 // one value per step (the reference's last_value / bootstrap_values pair).
 enum BootMode : int { kBootNone = 0, kBootRow = 1, kBootFull = 2 };
 
-// Address of boot(T-1) for `row` (g_zero when there is no bootstrap).
-template <class E>
-__device__ __forceinline__ const E* boot_last(const E* boot, int mode, int64_t row, int T) {
-  return mode == kBootFull ? boot + row * (int64_t)T + (T - 1)
-       : mode == kBootRow  ? boot + row
+// Where a thread's segment of S steps lies in the call's [E, T] arrays: how an op's load
+// reads an array's segment (seg) and finds one step of it (index).  RowAt: rows contiguous,
+// in one of the access modes above.
+template <int S_, int VEC>
+struct RowAt {
+  static constexpr int S = S_, kVec = VEC;
+  int64_t row;
+  int t0, T;
+  __device__ int64_t index(int t) const { return row * (int64_t)T + t; }
+  template <class E>
+  __device__ __forceinline__ void seg(const E* __restrict__ p, float (&v)[S]) const {
+    load_seg<S, VEC>(p + index(0), t0, T, v);
+  }
+};
+
+// ColumnAt: [T, E] in memory, steps ld elements apart; COLS environments side by side in a wave
+// (rlk_columns.hpp).  Steps beyond T read the last one.
+template <int S_, int COLS>
+struct ColumnAt {
+  static constexpr int S = S_, kVec = kElementAligned;
+  int64_t row;
+  int t0, T;
+  int64_t ld;
+  int64_t first_col;  // the wave's first environment, and how many it has
+  int cols;
+  __device__ int64_t index(int t) const { return row + t * ld; }
+  template <class E>
+  __device__ __forceinline__ void seg(const E* __restrict__ p, float (&v)[S]) const {
+    E raw[S];
+#pragma unroll
+    for (int i = 0; i < S; ++i) raw[i] = p[index(t0 + i < T ? t0 + i : T - 1)];
+#pragma unroll
+    for (int i = 0; i < S; ++i) v[i] = to_f32(raw[i]);
+  }
+};
+// Environments side by side in a wave (rows: one, of up to kWave lanes).
+template <class At>
+struct columns_of : std::integral_constant<int, kWave> {};
+template <int S, int COLS>
+struct columns_of<ColumnAt<S, COLS>> : std::integral_constant<int, COLS> {};
+
+// Address of boot(T-1) of the row (g_zero when there is no bootstrap).
+template <class At, class E>
+__device__ __forceinline__ const E* boot_last(const At& at, const E* boot, int mode) {
+  return mode == kBootFull ? boot + at.index(at.T - 1)
+       : mode == kBootRow  ? boot + at.row
                            : zero_src<E>();
 }
 
@@ -405,18 +447,17 @@ __device__ __forceinline__ const E* boot_last(const E* boot, int mode, int64_t r
 //   PER_STEP = false: the caller only uses boot(T-1) (no truncations), so only that value
 //                     is read (a per-step array at its last column);
 //   PER_STEP = true:  a per-step array is read in full; with a per-row value (or none) the
-//                     segment loads read `any_row` (any readable [T] row) and are discarded.
+//                     segment loads read `any` (another array of the call) and are discarded.
 // boot_prepare turns the raw registers into bt[i] = boot(t0 + i).
-template <int S, int VEC, bool PER_STEP, class E>
-__device__ __forceinline__ void boot_load(const E* __restrict__ boot, int mode, int64_t row,
-                                          int t0, int T, float (&seg)[S], float& last,
-                                          const E* any_row) {
+template <bool PER_STEP, class At, class E>
+__device__ __forceinline__ void boot_load(const At& at, const E* __restrict__ boot, int mode,
+                                          float (&seg)[At::S], float& last, const E* any) {
   if constexpr (PER_STEP) {
-    load_seg<S, VEC>(mode == kBootFull ? boot + row * (int64_t)T : any_row, t0, T, seg);
+    at.seg(mode == kBootFull ? boot : any, seg);
     // a per-step array already holds boot(T-1) in the segment that contains T-1
-    last = mode == kBootFull ? 0.f : to_f32(*boot_last(boot, mode, row, T));
+    last = mode == kBootFull ? 0.f : to_f32(*boot_last(at, boot, mode));
   } else {
-    last = to_f32(*boot_last(boot, mode, row, T));
+    last = to_f32(*boot_last(at, boot, mode));
   }
 }
 template <int S, bool PER_STEP>
@@ -430,14 +471,14 @@ __device__ __forceinline__ void boot_prepare(int mode, int t0, int T, float (&bt
 
 // The row's carry x[T] (backward) / x[-1] (forward): op.row_carry_src() gives its address,
 // nullptr for 0.
-// Ops whose map is not Affine give their row's carried state by op.row_state(row, T).
-template <class Op>
-__device__ __forceinline__ typename Op::Map::State row_carry(const Op& op, int64_t row, int T) {
+// Ops whose map is not Affine give their row's carried state by op.row_state(at).
+template <class Op, class At>
+__device__ __forceinline__ typename Op::Map::State row_carry(const Op& op, const At& at) {
   if constexpr (std::is_same<typename Op::Map, Affine>::value) {
-    const auto* src = op.row_carry_src(row, T);
+    const auto* src = op.row_carry_src(at);
     return src ? to_f32(*src) : 0.f;
   } else {
-    return op.row_state(row, T);
+    return op.row_state(at);
   }
 }
 
@@ -597,8 +638,9 @@ __device__ __forceinline__ double wave_total(double v) {
 
 // Every thread of the workgroup calls this once; thread 0 writes
 // partials[kStatWords*blockIdx.x + {0,1,2}] = {n, sum, sum of squares}.
+// (waves: the workgroup's, where it may have fewer than NT threads).
 template <int NT>
-__device__ __forceinline__ void block_stats(Stats st, double* __restrict__ partials) {
+__device__ __forceinline__ void block_stats(Stats st, double* __restrict__ partials, int waves = NT / kWave) {
   constexpr int NW = NT / kWave;
   __shared__ double s_st[kStatWords][NW];
   st.n = wave_total(st.n);
@@ -613,7 +655,7 @@ __device__ __forceinline__ void block_stats(Stats st, double* __restrict__ parti
   __syncthreads();
   if (threadIdx.x < kStatWords) {
     double a = 0.0;
-    for (int w = 0; w < NW; ++w) a += s_st[threadIdx.x][w];
+    for (int w = 0; w < waves; ++w) a += s_st[threadIdx.x][w];
     partials[kStatWords * blockIdx.x + threadIdx.x] = a;
   }
 }
@@ -820,14 +862,15 @@ __global__ __launch_bounds__(NT) void rows_kernel(const Op op, int64_t E, int T,
   const int64_t row = active ? row_id : E - 1;  // idle lanes of the last workgroup read a real row
   const int t0 = (FWD ? li : L - 1 - li) * S;
 
+  const RowAt<S, VEC> at{row, t0, T};
   Regs R;
-  op.template load<S, VEC>(row, t0, T, R);
+  op.load(at, R);
   // the first lane of a wave that is not the first of its row reads the neighbour step
   Halo edge{};
   if constexpr (HAS_HALO) {
-    if (lane == 0 && li > 0) edge = op.halo_load(row, clamp_step(FWD ? t0 - 1 : t0 + S, T), T);
+    if (lane == 0 && li > 0) edge = op.halo_load(at, clamp_step(FWD ? t0 - 1 : t0 + S, T), R);
   }
-  State carry = row_carry(op, row, T);
+  State carry = row_carry(op, at);
   op.template prepare<S, VEC>(R, row, t0, T);
   Halo h{};
   if constexpr (HAS_HALO) {
@@ -887,6 +930,7 @@ __global__ __launch_bounds__(NT) void rows_pair_kernel(const Op op, int64_t E, i
   const int lane = __lane_id();
   const int li = tid & (L - 1);  // position in scan order
   const int t0 = (FWD ? li : L - 1 - li) * S;
+  using At = RowAt<S, kAligned>;
   int64_t row[RPT];
   bool active[RPT];
   Regs R[RPT];
@@ -895,16 +939,16 @@ __global__ __launch_bounds__(NT) void rows_pair_kernel(const Op op, int64_t E, i
     const int64_t row_id = ((int64_t)blockIdx.x * RPT + u) * (NT >> log2L) + (tid >> log2L);
     active[u] = row_id < E;
     row[u] = active[u] ? row_id : E - 1;  // idle lanes of the last workgroup read a real row
-    op.template load<S, kAligned>(row[u], t0, T, R[u]);
+    op.load(At{row[u], t0, T}, R[u]);
   }
   Halo edge{};
   if constexpr (HAS_HALO) {
-    if (lane == 0 && li > 0) edge = op.halo_load(row[0], clamp_step(FWD ? t0 - 1 : t0 + S, T), T);
+    if (lane == 0 && li > 0) edge = op.halo_load(At{row[0], t0, T}, clamp_step(FWD ? t0 - 1 : t0 + S, T), R[0]);
   }
   State carry[RPT];
 #pragma unroll
   for (int u = 0; u < RPT; ++u) {
-    carry[u] = row_carry(op, row[u], T);
+    carry[u] = row_carry(op, At{row[u], t0, T});
     op.template prepare<S, kAligned>(R[u], row[u], t0, T);
   }
   Halo h[RPT];
@@ -1250,16 +1294,17 @@ __global__ __launch_bounds__(NT) void rows_strided_kernel(const Op op, int64_t E
   const int wbase = (FWD ? wave : NW - 1 - wave) * WSTEPS;
   const int lt = FWD ? lane : kWave - 1 - lane;
   auto seg_t0 = [&](int r) { return wbase + ((FWD ? r : Q - 1 - r) * kWave + lt) * S; };
+  auto seg_at = [&](int r) { return RowAt<S, VEC>{row, seg_t0(r), T}; };
 
   Regs R[Q];
 #pragma unroll
-  for (int r = 0; r < Q; ++r) op.template load<S, VEC>(row, seg_t0(r), T, R[r]);
+  for (int r = 0; r < Q; ++r) op.load(seg_at(r), R[r]);
   Halo edge{};
   if constexpr (HAS_HALO) {
     if (lane == 0 && (FWD ? wbase > 0 : wbase + WSTEPS < T))
-      edge = op.halo_load(row, clamp_step(FWD ? wbase - 1 : wbase + WSTEPS, T), T);
+      edge = op.halo_load(seg_at(0), clamp_step(FWD ? wbase - 1 : wbase + WSTEPS, T), R[0]);
   }
-  State carry = row_carry(op, row, T);
+  State carry = row_carry(op, seg_at(0));
 #pragma unroll
   for (int r = 0; r < Q; ++r) op.template prepare<S, VEC>(R[r], row, seg_t0(r), T);
 
@@ -1316,6 +1361,7 @@ __global__ __launch_bounds__(NT) void chain_kernel(const Op op, int64_t E, int T
   constexpr int WSTEPS = Q * kWave * kSeg;  // steps per wave chunk
   static_assert(NT % kWave == 0, "whole waves");
   using Regs = typename Op::template Regs<kSeg>;
+  using At = RowAt<kSeg, VEC>;
   using Halo = typename Op::Halo;
   using Map = typename Op::Map;
   using State = typename Map::State;
@@ -1419,14 +1465,14 @@ __global__ __launch_bounds__(NT) void chain_kernel(const Op op, int64_t E, int T
       // loads: Q segments, plus the neighbour step before the chunk in scan order
       Regs R[Q];
 #pragma unroll
-      for (int r = 0; r < Q; ++r) op.template load<kSeg, VEC>(row, seg_t0(r), T, R[r]);
+      for (int r = 0; r < Q; ++r) op.load(At{row, seg_t0(r), T}, R[r]);
       Halo edge{};
       if constexpr (HAS_HALO) {
         if (lane == 0 && (FWD ? wbase > 0 : wbase + WSTEPS < T))
-          edge = op.halo_load(row, clamp_step(FWD ? wbase - 1 : wbase + WSTEPS, T), T);
+          edge = op.halo_load(At{row, wbase, T}, clamp_step(FWD ? wbase - 1 : wbase + WSTEPS, T), R[0]);
       }
       const bool first = FWD ? (k == 0) : (k == tiles_per_row - 1);
-      State rc = (first && wave == 0) ? row_carry(op, row, T) : State{};
+      State rc = (first && wave == 0) ? row_carry(op, At{row, wbase, T}) : State{};
       [[maybe_unused]] Regs Rp;  // kPhased: the steps ahead of the row's tiles (below)
       if (it == 0 && tid == 0 && chained) {  // the epoch load was issued before the tile's loads
         s_epoch = (uint32_t)e_raw & kEpochMask;
@@ -1466,10 +1512,11 @@ __global__ __launch_bounds__(NT) void chain_kernel(const Op op, int64_t E, int T
         // load's latency (prefix sum [8,2^20-1] 20.59 -> 19.55 us, GAE [64,40001]
         // 19.41 -> 17.52 us on MI355X).
         if (first && wave == 0 && pre_live) {
-          op.template load<kSeg, VEC>(row, pre_t0, T, Rp);
+          const At pre_at{row, pre_t0, T};
+          op.load(pre_at, Rp);
           op.template prepare<kSeg, VEC>(Rp, row, pre_t0, T);
           Halo hp{};
-          if constexpr (HAS_HALO) hp = op.halo_load(row, clamp_step(FWD ? pre_t0 - 1 : pre_t0 + kSeg, T), T);
+          if constexpr (HAS_HALO) hp = op.halo_load(pre_at, clamp_step(FWD ? pre_t0 - 1 : pre_t0 + kSeg, T), Rp);
           Map sp[kSeg];
           op.template coef<kSeg, VEC>(Rp, hp, row, pre_t0, T, sp);
           State xp[kSeg];

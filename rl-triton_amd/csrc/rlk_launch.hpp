@@ -233,6 +233,35 @@ LongShape long_shape(int64_t E, int64_t T) {
   return r;
 }
 
+// Ops whose time is their action rows, not the [E, T] arrays (Retrace with any action count:
+// at 18 actions the rows are 84% of the call's bytes): one form of each launch only,
+// element-aligned with a run-time scan width, an eighth of the kernels of the other ops.
+template <class Op>
+struct one_form : std::false_type {};
+template <bool TRUNC, class E>
+struct one_form<RetraceOp<0, TRUNC, E>> : std::true_type {};
+
+// Dynamic LDS of a launch with `threads` threads per workgroup.
+template <class Op>
+size_t dynamic_lds(const Op&, int) { return 0; }
+template <bool TRUNC, class E>
+size_t dynamic_lds(const RetraceOp<0, TRUNC, E>& op, int threads) {
+  return (size_t)(threads / kWave) * action_stage_bytes(op.A);
+}
+
+// Such calls of few steps hold one step per thread, in rows of up to 512 steps: four times the
+// waves, each with one block of 64 action rows instead of four in turn.  It pays while the
+// waves are few enough to start at once; with more, four steps per thread keep the loads of the
+// next rows in flight.  Measured on MI355X (us, four steps -> one, float32 / bfloat16): A = 18
+// [64,64] 6.57 -> 3.50 / 7.34 -> 3.65, [300,250] 7.19 -> 5.18 / 7.88 -> 4.60, [1024,250] 10.03
+// -> 10.76 / 9.42 -> 8.73, [4096,128] 16.02 -> 18.40 / 11.61 -> 12.85; A = 6 [64,64] 4.54 ->
+// 2.88, [1024,250] 6.53 -> 7.26 / 7.20 -> 6.17.
+template <class Op>
+bool step_per_thread(int64_t E, int64_t T) {
+  if constexpr (!one_form<Op>::value) return false;
+  return T <= kNTWide && E * T <= 8 * kWave * (int64_t)device_cus();  // 8 waves per CU
+}
+
 // Workgroups of the launch that launch() makes for Op at [E, T] (E, T > 0).
 template <class Op>
 int64_t launch_grid(int64_t E, int64_t T) {
@@ -241,6 +270,7 @@ int64_t launch_grid(int64_t E, int64_t T) {
     return chain_grid(E, T, sh.threads, sh.segments);
   }
   if (rows_seg(T) == 1) return rows_grid(E, T, 1, kNT);
+  if (step_per_thread<Op>(E, T)) return rows_grid(E, T, 1, T <= kNT ? kNT : kNTWide);
   return rows_grid(E, T, 4, rows_threads(E, T));
 }
 
@@ -255,7 +285,7 @@ int64_t launch_grid(int64_t E, int64_t T) {
 template <class Op>
 struct paired_rows : std::false_type {};
 template <int NA, bool TRUNC>
-struct paired_rows<RetraceOp<NA, TRUNC, float>> : std::true_type {};
+struct paired_rows<RetraceOp<NA, TRUNC, float>> : std::bool_constant<(NA > 0)> {};
 
 template <class Op, int NT, int S, int VEC, int SP>
 hipError_t launch_rows(const Op& op, int64_t E, int T, hipStream_t stream) {
@@ -271,12 +301,12 @@ hipError_t launch_rows(const Op& op, int64_t E, int T, hipStream_t stream) {
       return hipLaunchKernel(k, dim3((unsigned)grid), dim3(NT / 2), args, 0, stream);
     }
   }
-  if constexpr (S == 4) {
+  if constexpr (S == 4 && !one_form<Op>::value) {
     if (log2L == 4) k = reinterpret_cast<const void*>(&rows_kernel<Op, NT, S, VEC, 16, SP>);
     else if (log2L == 5) k = reinterpret_cast<const void*>(&rows_kernel<Op, NT, S, VEC, 32, SP>);
     else if (log2L >= 6) k = reinterpret_cast<const void*>(&rows_kernel<Op, NT, S, VEC, kWave, SP>);
   }
-  return hipLaunchKernel(k, dim3((unsigned)grid), dim3(NT), args, 0, stream);
+  return hipLaunchKernel(k, dim3((unsigned)grid), dim3(NT), args, dynamic_lds(op, NT), stream);
 }
 
 // Aligned rows of 1025..2048 steps: one row per 256-thread workgroup, two wave-strided
@@ -302,7 +332,7 @@ hipError_t launch_strided(const Op& op, int64_t E, int T, hipStream_t stream) {
   int unused = 0;
   void* args[] = {const_cast<Op*>(&op), &E, &T, &unused};
   return hipLaunchKernel(reinterpret_cast<const void*>(&rows_strided_kernel<Op, kStridedThreads, kStridedSegments, kAligned, SP>),
-                         dim3((unsigned)E), dim3(kStridedThreads), args, 0, stream);
+                         dim3((unsigned)E), dim3(kStridedThreads), args, dynamic_lds(op, kStridedThreads), stream);
 }
 
 // Look-back poll budgets (rlk_debug_lookback): polls before a wait gives up (~1 s), and
@@ -343,7 +373,7 @@ hipError_t launch_chain(const Op& op, int64_t E, int T, uint64_t* ws, hipStream_
   void* args[] = {const_cast<Op*>(&op), &E, &T, &tpr, &ws, &fb, &spin_limit, &fallback_polls,
                   &row_major, &phase0};
   return hipLaunchKernel(reinterpret_cast<const void*>(&chain_kernel<Op, NT, Q, VEC, SP>),
-                         dim3((unsigned)grid), dim3(NT), args, 0, stream);
+                         dim3((unsigned)grid), dim3(NT), args, dynamic_lds(op, NT), stream);
 }
 
 template <class Op, int VEC, int SP>
@@ -412,7 +442,7 @@ enum class Kernel { kRows, kStrided, kChain };
 template <class Op, Kernel K>
 struct store_policies {
   static constexpr bool kBf16 = std::is_same<typename Op::Elem, bf16>::value;
-  static constexpr bool kWriteThrough = kBf16 || K != Kernel::kChain || long_rows_write_through<Op>::value;
+  static constexpr bool kWriteThrough = kBf16 || (K != Kernel::kChain && !one_form<Op>::value) || long_rows_write_through<Op>::value;
   static constexpr bool kNonTemporal = !kBf16 && K != Kernel::kStrided;
   static_assert(kWriteThrough || kNonTemporal, "some store policy");
 };
@@ -586,7 +616,7 @@ int launch(const Op& op, int64_t E, int64_t T, bool vec, void* workspace, size_t
   }
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   const int Ti = (int)T;
-  hipError_t e;
+  hipError_t e = hipErrorInvalidValue;
   if (T > kShortMaxT) {
     uint64_t* ws = reinterpret_cast<uint64_t*>(workspace);
     if (ws == nullptr || workspace_bytes_given < workspace_bytes(E, T) || !aligned16(ws))
@@ -597,22 +627,34 @@ int launch(const Op& op, int64_t E, int64_t T, bool vec, void* workspace, size_t
       if constexpr (phased_rows<Op>::value) {
         if (phased) return launch_long<Op, kPhased, SP>(op, E, Ti, ws, s, phase0);
       }
-      return vec ? launch_long<Op, kAligned, SP>(op, E, Ti, ws, s, 0)
-                 : launch_long<Op, kElementAligned, SP>(op, E, Ti, ws, s, 0);
+      if constexpr (!one_form<Op>::value) {
+        if (vec) return launch_long<Op, kAligned, SP>(op, E, Ti, ws, s, 0);
+      }
+      return launch_long<Op, kElementAligned, SP>(op, E, Ti, ws, s, 0);
     });
   } else if (strided_rows<Op>::value && vec && T > kShortMaxT / 2) {
-    e = dispatch_store_policy<Op, Kernel::kStrided>(E, T, [&](auto sp) {
-      return launch_strided<Op, decltype(sp)::value>(op, E, Ti, s);
-    });
+    if constexpr (strided_rows<Op>::value) {
+      e = dispatch_store_policy<Op, Kernel::kStrided>(E, T, [&](auto sp) {
+        return launch_strided<Op, decltype(sp)::value>(op, E, Ti, s);
+      });
+    }
   } else {
     e = dispatch_store_policy<Op, Kernel::kRows>(E, T, [&](auto sp) {
       constexpr int SP = decltype(sp)::value;
       if (rows_seg(T) == 1) return launch_rows<Op, kNT, 1, kElementAligned, SP>(op, E, Ti, s);
-      if (rows_threads(E, T) == kNT)
-        return vec ? launch_rows<Op, kNT, 4, kAligned, SP>(op, E, Ti, s)
-                   : launch_rows<Op, kNT, 4, kElementAligned, SP>(op, E, Ti, s);
-      return vec ? launch_rows<Op, kNTWide, 4, kAligned, SP>(op, E, Ti, s)
-                 : launch_rows<Op, kNTWide, 4, kElementAligned, SP>(op, E, Ti, s);
+      if constexpr (one_form<Op>::value) {
+        if (step_per_thread<Op>(E, T))
+          return T <= kNT ? launch_rows<Op, kNT, 1, kElementAligned, SP>(op, E, Ti, s)
+                          : launch_rows<Op, kNTWide, 1, kElementAligned, SP>(op, E, Ti, s);
+      }
+      const bool narrow = rows_threads(E, T) == kNT;
+      if constexpr (!one_form<Op>::value) {
+        if (vec)
+          return narrow ? launch_rows<Op, kNT, 4, kAligned, SP>(op, E, Ti, s)
+                        : launch_rows<Op, kNTWide, 4, kAligned, SP>(op, E, Ti, s);
+      }
+      return narrow ? launch_rows<Op, kNT, 4, kElementAligned, SP>(op, E, Ti, s)
+                    : launch_rows<Op, kNTWide, 4, kElementAligned, SP>(op, E, Ti, s);
     });
   }
   return e == hipSuccess ? RLK_OK : RLK_ERR_LAUNCH;

@@ -52,15 +52,14 @@ struct GaeOp {
     float blast;
   };
 
-  template <int S, int VEC>
-  __device__ void load(int64_t row, int t0, int T, Regs<S>& R) const {
-    const int64_t o = row * (int64_t)T;
-    load_seg<S, VEC>(r + o, t0, T, R.r);
-    load_seg<S, VEC>(v + o, t0, T, R.v);
-    load_seg<S, VEC>(term + o, t0, T, R.te);
-    if constexpr (TRUNC) load_seg<S, VEC>(trunc + o, t0, T, R.tr);
+  template <class At>
+  __device__ void load(const At& at, Regs<At::S>& R) const {
+    at.seg(r, R.r);
+    at.seg(v, R.v);
+    at.seg(term, R.te);
+    if constexpr (TRUNC) at.seg(trunc, R.tr);
     else fill_regs(R.tr, 0.f);
-    boot_load<S, VEC, TRUNC>(boot, boot_mode, row, t0, T, R.bt, R.blast, r + o);
+    boot_load<TRUNC>(at, boot, boot_mode, R.bt, R.blast, r);
   }
   template <int S, int VEC>
   __device__ void prepare(Regs<S>& R, int64_t, int t0, int T) const {
@@ -68,7 +67,8 @@ struct GaeOp {
   }
   template <int S>
   __device__ float export_first(const Regs<S>& R) const { return R.v[0]; }
-  __device__ float halo_load(int64_t row, int t, int T) const { return to_f32(v[row * (int64_t)T + t]); }
+  template <class At>
+  __device__ float halo_load(const At& at, int t, const Regs<At::S>&) const { return to_f32(v[at.index(t)]); }
 
   template <int S, int VEC = kElementAligned>
   __device__ void coef(const Regs<S>& R, float vh, int64_t, int t0, int T, Affine (&m)[S]) const {
@@ -90,7 +90,8 @@ struct GaeOp {
       m[i].mul = in ? gl * (1.f - done) : 1.f;
     }
   }
-  __device__ const E* row_carry_src(int64_t, int) const { return nullptr; }
+  template <class At>
+  __device__ const E* row_carry_src(const At&) const { return nullptr; }
 
   template <int S, int VEC, int SP = 0>
   __device__ void emit(const Regs<S>&, float, const float (&xs)[S], float, int64_t row, int t0,
@@ -176,16 +177,15 @@ struct MaskedGaeOp {
     float blast;
   };
 
-  template <int S, int VEC>
-  __device__ void load(int64_t row, int t0, int T, Regs<S>& R) const {
-    const int64_t o = row * (int64_t)T;
-    load_seg<S, VEC>(r + o, t0, T, R.r);
-    load_seg<S, VEC>(v + o, t0, T, R.v);
-    load_seg<S, VEC>(term + o, t0, T, R.te);
-    load_seg<S, VEC>(mask + o, t0, T, R.mk);
+  template <class At>
+  __device__ void load(const At& at, Regs<At::S>& R) const {
+    at.seg(r, R.r);
+    at.seg(v, R.v);
+    at.seg(term, R.te);
+    at.seg(mask, R.mk);
     if constexpr (TRUNC) {
-      load_seg<S, VEC>(trunc + o, t0, T, R.tr);
-      boot_load<S, VEC, true>(boot, boot_mode, row, t0, T, R.bt, R.blast, r + o);
+      at.seg(trunc, R.tr);
+      boot_load<true>(at, boot, boot_mode, R.bt, R.blast, r);
     } else {
       fill_regs(R.tr, 0.f), fill_regs(R.bt, 0.f);
       R.blast = 0.f;
@@ -196,8 +196,9 @@ struct MaskedGaeOp {
     if constexpr (TRUNC) boot_prepare<S, true>(boot_mode, t0, T, R.bt, R.blast);
   }
   // state after the row: next value boot(T-1), advantage 0
-  __device__ NvX row_state(int64_t row, int T) const {
-    return NvX{to_f32(*boot_last(boot, boot_mode, row, T)), 0.f};
+  template <class At>
+  __device__ NvX row_state(const At& at) const {
+    return NvX{to_f32(*boot_last(at, boot, boot_mode)), 0.f};
   }
 
   template <int S, int VEC = kElementAligned>
@@ -298,17 +299,16 @@ struct VtraceOp {
     float blast;
   };
 
-  template <int S, int VEC>
-  __device__ void load(int64_t row, int t0, int T, Regs<S>& R) const {
-    const int64_t o = row * (int64_t)T;
-    load_seg<S, VEC>(lpt + o, t0, T, R.rho);
-    load_seg<S, VEC>(lpb + o, t0, T, R.c);
-    load_seg<S, VEC>(v + o, t0, T, R.v);
-    load_seg<S, VEC>(r + o, t0, T, R.r);
-    load_seg<S, VEC>(term + o, t0, T, R.te);
-    if constexpr (TRUNC) load_seg<S, VEC>(trunc + o, t0, T, R.tr);
+  template <class At>
+  __device__ void load(const At& at, Regs<At::S>& R) const {
+    at.seg(lpt, R.rho);
+    at.seg(lpb, R.c);
+    at.seg(v, R.v);
+    at.seg(r, R.r);
+    at.seg(term, R.te);
+    if constexpr (TRUNC) at.seg(trunc, R.tr);
     else fill_regs(R.tr, 0.f);
-    boot_load<S, VEC, TRUNC>(boot, boot_mode, row, t0, T, R.bt, R.blast, r + o);
+    boot_load<TRUNC>(at, boot, boot_mode, R.bt, R.blast, r);
   }
   template <int S, int VEC>
   __device__ void prepare(Regs<S>& R, int64_t, int t0, int T) const {
@@ -324,7 +324,8 @@ struct VtraceOp {
   }
   template <int S>
   __device__ float export_first(const Regs<S>& R) const { return R.v[0]; }
-  __device__ float halo_load(int64_t row, int t, int T) const { return to_f32(v[row * (int64_t)T + t]); }
+  template <class At>
+  __device__ float halo_load(const At& at, int t, const Regs<At::S>&) const { return to_f32(v[at.index(t)]); }
 
   // continuation value at step t from the raw next-step value (values or targets)
   // last: t == T - 1
@@ -347,7 +348,8 @@ struct VtraceOp {
       m[i].mul = in ? gamma * R.c[i] * (1.f - done) : 1.f;
     }
   }
-  __device__ const E* row_carry_src(int64_t, int) const { return nullptr; }
+  template <class At>
+  __device__ const E* row_carry_src(const At&) const { return nullptr; }
 
   template <int S, int VEC, int SP = 0>
   __device__ void emit(const Regs<S>& R, float vh, const float (&xs)[S], float x_next, int64_t row,
@@ -369,12 +371,291 @@ struct VtraceOp {
 };
 
 // ------------------------------------------------------------------------------------------
+// Action rows of any length A, reduced by a wave through LDS.
+//
+// A wave's segments are a contiguous run of steps, so their action rows are a contiguous run
+// of words in pi and in nq.  Each lane reading its own steps' rows touches 64 cache lines per
+// load, each line again by later loads, and the lines do not stay in L1 (A = 18: two arrays of
+// 18 KB per wave): Retrace then ran at a quarter of the streaming rate.  Here the wave takes
+// the run 64 rows at a time: word j*64 + lane of them goes to lane `lane` (each load 256
+// contiguous bytes; bfloat16: pairs), from there to LDS at a row stride of A | 1 words (odd: the 64
+// rows start in different banks), and lane l sums row l in order of the actions, the order
+// (and the bits) of a loop over the row.  The next 64 rows' loads are issued before the sums.
+// Short rows go 128 or 256 at a time (bfloat16 A = 6 [1024,250] 6.7 us at 64 rows), rows of
+// more than kPipedActions actions in slices of 16 actions.
+//
+// Bound by HBM: on MI355X, float32, lane-by-lane rows -> this: A = 18 [4096,128] 78.3 -> 15.8
+// us (94 MB, 6.0 TB/s), [256,2048] 138.6 -> 16.8, [64,8192] 115.5 -> 23.8; A = 6 [4096,128]
+// 23.9 -> 8.6; bfloat16 A = 18 [4096,128] 108.1 -> 11.5.  A branch around each load or LDS
+// read instead of the straight-line batches took 28.4 us at A = 18 [4096,128].
+//
+// LDS is the wave's own, dynamic (action_stage_bytes per wave): no barrier.
+// ------------------------------------------------------------------------------------------
+constexpr int kPipedActions = 18, kActionSlice = 16;
+// Four bytes from an element's address on: one float, or a pair of bfloat16.
+typedef uint32_t ua_u1 __attribute__((aligned(2)));
+__device__ __forceinline__ uint32_t load_word_ua(const float* p) { return __float_as_uint(*p); }
+__device__ __forceinline__ uint32_t load_word_ua(const bf16* p) { return *reinterpret_cast<const ua_u1*>(p); }
+__host__ __device__ inline int action_stage_stride(int A) { return A <= kPipedActions ? (A | 1) : (kActionSlice | 1); }
+// Two staged arrays of 64 rows (rows of up to 9 actions: 128, up to 5: 256), the last row read
+// up to its batch's loads; later two result arrays of up to 256 steps.  At most 10 KB: sixteen
+// waves per CU.
+__host__ __device__ inline int action_stage_bytes(int A) {
+  const int rows = kWave * (A <= 5 ? 4 : A <= 9 ? 2 : 1);
+  const int batch = A <= 5 ? 5 : A <= 6 ? 6 : A <= 9 ? 9 : A <= 12 ? 12 : kPipedActions;
+  const int over = A < batch ? batch - A : 0;
+  const int b = (2 * rows * action_stage_stride(A) + over) * (int)sizeof(float);
+  return ((b < 2048 ? 2048 : b) + 15) & ~15;
+}
+
+// LDS accesses of one wave stay in program order across lanes.
+__device__ __forceinline__ void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
+// The run of steps that the wave's lanes hold, as step indexes of the [E, T] arrays.  Lanes
+// hold a row's segments in reverse (backward scans): the run starts at the last lane of the
+// first row and ends with the first lane of the last one.  (Lanes of rows past E repeat row
+// E - 1, whole.)
+template <class At>
+__device__ __forceinline__ void wave_run(const At& at, int64_t& first, int& steps) {
+  constexpr int S = At::S;
+  const int row_lo = __builtin_amdgcn_readfirstlane((int)(uint32_t)at.row);
+  const int row_hi = __builtin_amdgcn_readlane((int)(uint32_t)at.row, kWave - 1);
+  const int in_lo = __popcll(__ballot((int)(uint32_t)at.row == row_lo));
+  const int in_hi = __popcll(__ballot((int)(uint32_t)at.row == row_hi));
+  const int t_lo = __builtin_amdgcn_readlane(at.t0, in_lo - 1);
+  const int t_hi = __builtin_amdgcn_readlane(at.t0, kWave - in_hi) + S;
+  const int64_t base = (int64_t)lane0_u64((uint64_t)at.index(0));
+  first = base + t_lo;
+  steps = (int)(uint32_t)(row_hi - row_lo) * at.T + (t_hi < at.T ? t_hi : at.T) - t_lo;
+  if (steps < 0) steps = 0;
+}
+
+template <class At, class E>
+__device__ __forceinline__ void reduce_actions(const At& at, const E* __restrict__ pi,
+                                               const E* __restrict__ nq,
+                                               const int64_t* __restrict__ act, int A,
+                                               float (&enq)[At::S], float (&pa)[At::S],
+                                               float& pa_next) {
+  // Rows: the wave's run of steps, M * 64 of them per round.  Columns: step r of every chunk in
+  // round r, each chunk's COLS rows a contiguous piece; lane l's own step is row l.
+  constexpr int PIECE_ROWS = columns_of<At>::value;
+  constexpr bool COLUMNS = PIECE_ROWS < kWave;
+  constexpr int S = At::S, ROUNDS = S;
+  extern __shared__ float s_actions[];
+  const int lane = __lane_id();
+  const int stride = action_stage_stride(A);
+  float* sp = s_actions + (threadIdx.x / kWave) * (action_stage_bytes(A) / (int)sizeof(float));
+  int64_t first = 0;
+  int steps = kWave * S;
+  if constexpr (!COLUMNS) wave_run(at, first, steps);
+  // rows of round r's pieces of at most `most` rows, and the first one's step index
+  auto rows_of = [&](int r, int most) {
+    if constexpr (COLUMNS) return most < at.cols ? most : at.cols;
+    else return steps - r * most < most ? steps - r * most : most;
+  };
+  auto piece_of = [&](int r, int most, int piece) -> int64_t {
+    if constexpr (COLUMNS) {
+      const int t = __builtin_amdgcn_readlane(at.t0, piece * most) + r;
+      return at.first_col + (t < at.T ? t : at.T - 1) * at.ld;
+    } else {
+      return first + r * most;
+    }
+  };
+  // The step after the wave's (the row's next; step T - 1 again where there is none): its action
+  // is read ahead of the rows, its probability beside them, once the action is there.
+  int64_t next;
+  {
+    const int t = at.t0 + S < at.T ? at.t0 + S : at.T - 1;
+    if constexpr (COLUMNS) next = at.index(t);
+    else next = (int64_t)lane0_u64((uint64_t)at.index(t));
+  }
+  const int64_t a_next = act[next];
+  const E* p_next = pi + next * A + (a_next >= 0 && a_next < A ? a_next : 0);
+  E raw_next{};
+  float e[ROUNDS], p_taken[ROUNDS];
+#pragma unroll
+  for (int r = 0; r < ROUNDS; ++r) e[r] = p_taken[r] = 0.f;
+  auto keep = [&](int r, float s, float pt) {
+#pragma unroll
+    for (int k = 0; k < ROUNDS; ++k) {
+      e[k] = k == r ? s : e[k];
+      p_taken[k] = k == r ? pt : p_taken[k];
+    }
+  };
+  int Av = A;  // in a vector register: selects on it stay selects, not branches around reads
+  asm("" : "+v"(Av));
+  if (A <= kPipedActions) {
+    // B >= A loads per array and lane, straight-line code (a branch per load made the compiler
+    // wait at each): words past the run repeat its last one, sums past A are dropped.
+    auto rounds = [&](auto b, auto m) {
+      constexpr int B = decltype(b)::value;
+      constexpr int M = S == 1 || COLUMNS ? 1 : decltype(m)::value, ROWS = M * kWave;  // per round
+      constexpr int PR = COLUMNS ? PIECE_ROWS : ROWS, PIECES = ROWS / PR;  // rows per piece
+      constexpr int PK = 4 / (int)sizeof(E);  // elements per 4-byte load
+      constexpr int NL = (PR * B + PK * kWave - 1) / (PK * kWave);  // loads per lane and piece
+      float* sn = sp + ROWS * stride;
+      uint32_t vp[PIECES][NL], vn[PIECES][NL];
+      int64_t a_t[M];
+      // floor(w / A) for w < 2^11: (w * ceil(2^20 / A)) >> 20
+      const uint32_t magic = (A & 1) ? 0u : ((1u << 20) + (uint32_t)A - 1) / (uint32_t)A;
+      auto issue = [&](int r) {
+        const int rows = rows_of(r, PR), last = rows * A - PK;
+#pragma unroll
+        for (int k = 0; k < M; ++k) {
+          if constexpr (COLUMNS) {
+            a_t[k] = act[at.index(at.t0 + r < at.T ? at.t0 + r : at.T - 1)];
+          } else {
+            const int i = k * kWave + lane;
+            a_t[k] = act[first + r * ROWS + (i < rows ? i : rows - 1)];
+          }
+        }
+#pragma unroll
+        for (int c = 0; c < PIECES; ++c) {
+          const int64_t base = piece_of(r, PR, c) * A;
+#pragma unroll
+          for (int j = 0; j < NL; ++j) {
+            const int w = PK * (j * kWave + lane);
+            vp[c][j] = load_word_ua(pi + base + (w < last ? w : last));
+            vn[c][j] = load_word_ua(nq + base + (w < last ? w : last));
+          }
+        }
+      };
+      issue(0);
+#pragma unroll 1
+      for (int r = 0; r * ROWS < steps; ++r) {
+        int64_t at_r[M];
+#pragma unroll
+        for (int k = 0; k < M; ++k) at_r[k] = a_t[k];
+        const uint32_t end = rows_of(r, PR) * A;
+#pragma unroll
+        for (int c = 0; c < PIECES; ++c) {
+#pragma unroll
+          for (int j = 0; j < NL; ++j) {
+            const uint32_t w = PK * (j * kWave + lane);
+            // (whole waves of words: a scalar branch)
+            if (PK == 1 && PR % kWave == 0 ? j * kWave < PR * A : w < (uint32_t)(PR * A)) {
+              const uint32_t pos = c * PR * stride + w + ((w * magic) >> 20);
+              if constexpr (PK == 1) {
+                sp[pos] = __uint_as_float(vp[c][j]);
+                sn[pos] = __uint_as_float(vn[c][j]);
+              } else {
+                // a pair lies in one row, or (odd A) rows follow each other without a gap.  The
+                // run's last word alone was read with the one before it.
+                const bool alone = w + 1 == end;
+                const uint32_t up = alone ? vp[c][j] >> 16 : vp[c][j], un = alone ? vn[c][j] >> 16 : vn[c][j];
+                sp[pos] = __uint_as_float(up << 16);
+                sn[pos] = __uint_as_float(un << 16);
+                if (w + 1 < (uint32_t)(PR * A)) {
+                  sp[pos + 1] = __uint_as_float(up & 0xffff0000u);
+                  sn[pos + 1] = __uint_as_float(un & 0xffff0000u);
+                }
+              }
+            }
+          }
+        }
+        wave_lds_fence();
+        raw_next = *p_next;
+        if ((r + 1) * ROWS < steps) issue(r + 1);
+#pragma unroll
+        for (int k = 0; k < M; ++k) {
+          const int row = (k * kWave + lane) * stride;
+          float s = 0.f;
+#pragma unroll
+          for (int a = 0; a < B; ++a) {
+            const float t = fmaf(sp[row + a], sn[row + a], s);
+            s = a < Av ? t : s;
+          }
+          keep(r * M + k, s, at_r[k] >= 0 && at_r[k] < A ? sp[row + (int)at_r[k]] : 0.f);
+        }
+        wave_lds_fence();
+      }
+    };
+    if (steps > 0) {
+      using std::integral_constant;
+      if (A <= 5) rounds(integral_constant<int, 5>{}, integral_constant<int, 4>{});
+      else if (A == 6) rounds(integral_constant<int, 6>{}, integral_constant<int, 2>{});
+      else if (A <= 9) rounds(integral_constant<int, 9>{}, integral_constant<int, 2>{});
+      else if (A <= 12) rounds(integral_constant<int, 12>{}, integral_constant<int, 1>{});
+      else rounds(integral_constant<int, kPipedActions>{}, integral_constant<int, 1>{});
+    }
+  } else {
+    constexpr int PR = PIECE_ROWS;
+#pragma unroll 1
+    for (int r = 0; r * kWave < steps; ++r) {
+      const int rows = rows_of(r, PR);
+      int64_t a_t;
+      if constexpr (COLUMNS) a_t = act[at.index(at.t0 + r < at.T ? at.t0 + r : at.T - 1)];
+      else a_t = act[first + r * kWave + (lane < rows ? lane : rows - 1)];
+      raw_next = *p_next;
+      float* sn = sp + kWave * stride;
+      const int s_in = lane / kActionSlice, a_in = lane & (kActionSlice - 1);
+      float s = 0.f, pt = 0.f;
+#pragma unroll 1
+      for (int a0 = 0; a0 < A; a0 += kActionSlice) {
+        E vp[kActionSlice], vn[kActionSlice];
+        const int a = a0 + a_in < A ? a0 + a_in : A - 1;
+#pragma unroll
+        for (int j = 0; j < kActionSlice; ++j) {
+          const int sj = j * (kWave / kActionSlice) + s_in;  // row of the round
+          // (a load's four rows lie in one piece)
+          const int k = sj - (j * (kWave / kActionSlice)) / PR * PR;
+          const int64_t w = (piece_of(r, PR, (j * (kWave / kActionSlice)) / PR) + (k < rows ? k : rows - 1)) * A + a;
+          vp[j] = pi[w];
+          vn[j] = nq[w];
+        }
+#pragma unroll
+        for (int j = 0; j < kActionSlice; ++j) {
+          const int sj = j * (kWave / kActionSlice) + s_in;
+          sp[sj * stride + a_in] = to_f32(vp[j]);
+          sn[sj * stride + a_in] = to_f32(vn[j]);
+        }
+        wave_lds_fence();
+#pragma unroll
+        for (int k = 0; k < kActionSlice; ++k) {
+          const float t = fmaf(sp[lane * stride + k], sn[lane * stride + k], s);
+          s = a0 + k < Av ? t : s;
+        }
+        const int64_t k_t = a_t - a0;
+        if (k_t >= 0 && k_t < kActionSlice && a_t < A) pt = sp[lane * stride + (int)k_t];
+        wave_lds_fence();
+      }
+      keep(r, s, pt);
+    }
+  }
+  pa_next = a_next >= 0 && a_next < A ? to_f32(raw_next) : 0.f;
+  if constexpr (COLUMNS) {
+#pragma unroll
+    for (int i = 0; i < S; ++i) enq[i] = e[i], pa[i] = p_taken[i];
+    return;
+  }
+  // from "lane l has steps l, 64 + l, ..." of the run to each lane's own segment
+#pragma unroll
+  for (int r = 0; r < ROUNDS; ++r) {
+    sp[r * kWave + lane] = e[r];
+    sp[(ROUNDS + r) * kWave + lane] = p_taken[r];
+  }
+  wave_lds_fence();
+  const int local = (int)(at.index(at.t0) - first);
+#pragma unroll
+  for (int i = 0; i < S; ++i) {
+    const int k = local + i < ROUNDS * kWave ? local + i : ROUNDS * kWave - 1;  // padding: any
+    enq[i] = sp[k < 0 ? 0 : k];
+    pa[i] = sp[ROUNDS * kWave + (k < 0 ? 0 : k)];
+  }
+  wave_lds_fence();
+}
+
+// ------------------------------------------------------------------------------------------
 // Retrace(lambda): kernels/retrace_fused.py:116-201 (retrace_fused_kernel).
 //   E_pi[Q'] = sum_a pi[t,a]*nq[t,a];  pi_a = pi[t, a_t] (0 if a_t outside [0, A))
 //   rho = min(pi_a/mu, rho_bar),  c = lambda*min(pi_a/mu, c_bar)
 //   add = r + gamma*E_pi[Q']*(1-term) - q,  mul = gamma*c[t+1]*(1-done),  c[T] = 0
 //   Q_ret = x + q;  advantages = rho*(r + gamma*Q_ret[t+1]*(1-term) - q),  Q_ret[T] = 0
-// NA > 0: compile-time action count (vector loads of the [S, A] block); NA == 0: runtime A.
+// NA > 0: compile-time action count (vector loads of the [S, A] block); NA == 0: any A
+// (reduce_actions).
 // ------------------------------------------------------------------------------------------
 template <int NA, bool TRUNC, class E = float>
 struct RetraceOp {
@@ -401,78 +682,90 @@ struct RetraceOp {
   template <int S>
   struct Regs {
     float q[S], r[S], te[S], tr[S], rho[S], c[S], enq[S];
+    float pa_next;  // NA == 0: pi of the action taken at the step after the wave's (halo_load)
   };
 
-  // (rho, c, E_pi[Q']) at one step from its action row
+  // rho and c at one step from the probability of its action under both policies
+  __device__ __forceinline__ void clipped_ratios(float pa, float m, float& rho, float& c) const {
+    const float ratio = pa / m;
+    rho = fminf(ratio, rho_bar);
+    c = lambda * fminf(ratio, c_bar);
+  }
+
+  // (rho, c, E_pi[Q']) at one step from its action row (NA > 0)
   template <class P>
   __device__ __forceinline__ void step_terms(const P* p, const P* n, int64_t a_t, float m,
                                              float& rho, float& c, float& enq) const {
     float e = 0.f, pa = 0.f;
-    const int na = NA > 0 ? NA : A;
-    for (int a = 0; a < na; ++a) {
+#pragma unroll
+    for (int a = 0; a < NA; ++a) {
       const float pv = to_f32(p[a]);
       e = fmaf(pv, to_f32(n[a]), e);
       pa = (a == a_t) ? pv : pa;
     }
-    const float ratio = pa / m;
-    rho = fminf(ratio, rho_bar);
-    c = lambda * fminf(ratio, c_bar);
+    clipped_ratios(pa, m, rho, c);
     enq = e;
   }
 
   // Unlike the other ops, the [S, A] action blocks are reduced to (rho, c, E_pi[Q']) here,
   // at load time, so a segment holds three values per step instead of 2A.
-  template <int S, int VEC>
-  __device__ void load(int64_t row, int t0, int T, Regs<S>& R) const {
+  template <class At>
+  __device__ void load(const At& at, Regs<At::S>& R) const {
+    constexpr int S = At::S, VEC = At::kVec;
     static_assert(VEC != kPhased, "the [E, T, A] arrays have no common row phase");
-    const int64_t o = row * (int64_t)T;
+    const int t0 = at.t0, T = at.T;
     float m[S];
-    load_seg<S, VEC>(q + o, t0, T, R.q);
-    load_seg<S, VEC>(r + o, t0, T, R.r);
-    load_seg<S, VEC>(term + o, t0, T, R.te);
-    if constexpr (TRUNC) load_seg<S, VEC>(trunc + o, t0, T, R.tr);
+    at.seg(q, R.q);
+    at.seg(r, R.r);
+    at.seg(term, R.te);
+    if constexpr (TRUNC) at.seg(trunc, R.tr);
     else fill_regs(R.tr, 0.f);
-    load_seg<S, VEC>(mu + o, t0, T, m);
-    int64_t at[S];
-    if constexpr (VEC == kAligned) {
-      // a quad of actions is 32 contiguous bytes, 16-byte aligned (the launch checks the
-      // pointer): two 16-byte loads instead of four 8-byte ones (Retrace [4096,128]
-      // 6.60 -> 6.53 us on MI355X); a quad beyond T reads the row's last quad
-      typedef long long i64x2 __attribute__((ext_vector_type(2)));
+    at.seg(mu, m);
+    if constexpr (NA == 0) {
+      float pa[S];
+      reduce_actions(at, pi, nq, act, A, R.enq, pa, R.pa_next);
 #pragma unroll
-      for (int qd = 0; qd < S / 4; ++qd) {
-        const int t = t0 + 4 * qd;
-        const i64x2* pq = reinterpret_cast<const i64x2*>(act + o + (t < T ? t : T - 4));
-        const i64x2 u = pq[0], w = pq[1];
-        at[4 * qd] = u.x, at[4 * qd + 1] = u.y, at[4 * qd + 2] = w.x, at[4 * qd + 3] = w.y;
-      }
+      for (int i = 0; i < S; ++i) clipped_ratios(pa[i], m[i], R.rho[i], R.c[i]);
     } else {
+      int64_t a_t[S];
+      if constexpr (VEC == kAligned) {
+        // a quad of actions is 32 contiguous bytes, 16-byte aligned (the launch checks the
+        // pointer): two 16-byte loads instead of four 8-byte ones (Retrace [4096,128]
+        // 6.60 -> 6.53 us on MI355X); a quad beyond T reads the row's last quad
+        typedef long long i64x2 __attribute__((ext_vector_type(2)));
 #pragma unroll
-      for (int i = 0; i < S; ++i) at[i] = act[o + clamp_step(t0 + i, T)];
-    }
-    if constexpr (NA > 0 && VEC == kAligned && (S * NA) % 4 == 0 && S * NA <= 16) {
-      // the [S, NA] blocks are contiguous and 16-byte aligned; a quad beyond T reads the
-      // row's first quad instead.  (Larger blocks take the per-step path below: two tiles
-      // of them would not fit the register file.)
-      float pb[S * NA], nb[S * NA];
-      const E* pp = pi + (o + t0) * NA;
-      const E* np = nq + (o + t0) * NA;
+        for (int qd = 0; qd < S / 4; ++qd) {
+          const int t = t0 + 4 * qd;
+          const i64x2* pq = reinterpret_cast<const i64x2*>(act + at.index(t < T ? t : T - 4));
+          const i64x2 u = pq[0], w = pq[1];
+          a_t[4 * qd] = u.x, a_t[4 * qd + 1] = u.y, a_t[4 * qd + 2] = w.x, a_t[4 * qd + 3] = w.y;
+        }
+      } else {
 #pragma unroll
-      for (int qd = 0; qd < S * NA / 4; ++qd) {
-        const bool in = t0 + (4 * qd) / NA < T;
-        const float4 a4 = load_quad(in ? pp + 4 * qd : pi + o * NA);
-        const float4 b4 = load_quad(in ? np + 4 * qd : nq + o * NA);
-        pb[4 * qd] = a4.x, pb[4 * qd + 1] = a4.y, pb[4 * qd + 2] = a4.z, pb[4 * qd + 3] = a4.w;
-        nb[4 * qd] = b4.x, nb[4 * qd + 1] = b4.y, nb[4 * qd + 2] = b4.z, nb[4 * qd + 3] = b4.w;
+        for (int i = 0; i < S; ++i) a_t[i] = act[at.index(clamp_step(t0 + i, T))];
       }
+      if constexpr (VEC == kAligned && (S * NA) % 4 == 0 && S * NA <= 16) {
+        // the [S, NA] blocks are contiguous and 16-byte aligned; a quad beyond T reads the
+        // row's first quad instead.
+        float pb[S * NA], nb[S * NA];
+        const E* pp = pi + at.index(t0) * NA;
+        const E* np = nq + at.index(t0) * NA;
 #pragma unroll
-      for (int i = 0; i < S; ++i) step_terms(pb + i * NA, nb + i * NA, at[i], m[i], R.rho[i], R.c[i], R.enq[i]);
-    } else {
-      const int na = NA > 0 ? NA : A;
+        for (int qd = 0; qd < S * NA / 4; ++qd) {
+          const bool in = t0 + (4 * qd) / NA < T;
+          const float4 a4 = load_quad(in ? pp + 4 * qd : pi + at.index(0) * NA);
+          const float4 b4 = load_quad(in ? np + 4 * qd : nq + at.index(0) * NA);
+          pb[4 * qd] = a4.x, pb[4 * qd + 1] = a4.y, pb[4 * qd + 2] = a4.z, pb[4 * qd + 3] = a4.w;
+          nb[4 * qd] = b4.x, nb[4 * qd + 1] = b4.y, nb[4 * qd + 2] = b4.z, nb[4 * qd + 3] = b4.w;
+        }
 #pragma unroll
-      for (int i = 0; i < S; ++i) {
-        const int64_t base = (o + clamp_step(t0 + i, T)) * na;
-        step_terms(pi + base, nq + base, at[i], m[i], R.rho[i], R.c[i], R.enq[i]);
+        for (int i = 0; i < S; ++i) step_terms(pb + i * NA, nb + i * NA, a_t[i], m[i], R.rho[i], R.c[i], R.enq[i]);
+      } else {
+#pragma unroll
+        for (int i = 0; i < S; ++i) {
+          const int64_t base = at.index(clamp_step(t0 + i, T)) * NA;
+          step_terms(pi + base, nq + base, a_t[i], m[i], R.rho[i], R.c[i], R.enq[i]);
+        }
       }
     }
   }
@@ -480,11 +773,12 @@ struct RetraceOp {
   __device__ void prepare(Regs<S>&, int64_t, int, int) const {}
   template <int S>
   __device__ Halo2 export_first(const Regs<S>& R) const { return Halo2{R.c[0], R.q[0]}; }
-  __device__ Halo2 halo_load(int64_t row, int t, int T) const {
-    const int64_t i = row * (int64_t)T + t;
-    const int na = NA > 0 ? NA : A;
+  template <class At>
+  __device__ Halo2 halo_load(const At& at, int t, const Regs<At::S>& R) const {
+    const int64_t i = at.index(t);
     float rho, c, enq;
-    step_terms(pi + i * na, nq + i * na, act[i], to_f32(mu[i]), rho, c, enq);
+    if constexpr (NA == 0) clipped_ratios(R.pa_next, to_f32(mu[i]), rho, c);
+    else step_terms(pi + i * NA, nq + i * NA, act[i], to_f32(mu[i]), rho, c, enq);
     return Halo2{c, to_f32(q[i])};
   }
 
@@ -502,7 +796,8 @@ struct RetraceOp {
       m[i].mul = in ? gamma * c_next * (1.f - done) : 1.f;
     }
   }
-  __device__ const E* row_carry_src(int64_t, int) const { return nullptr; }
+  template <class At>
+  __device__ const E* row_carry_src(const At&) const { return nullptr; }
 
   template <int S, int VEC, int SP = 0>
   __device__ void emit(const Regs<S>& R, Halo2 h, const float (&xs)[S], float x_next, int64_t row,
@@ -557,16 +852,15 @@ struct ReturnsOp {
     float blast;
   };
 
-  template <int S, int VEC>
-  __device__ void load(int64_t row, int t0, int T, Regs<S>& R) const {
-    const int64_t o = row * (int64_t)T;
-    load_seg<S, VEC>(r + o, t0, T, R.r);
-    if constexpr (NV) load_seg<S, VEC>(nv + o, t0, T, R.nv);
+  template <class At>
+  __device__ void load(const At& at, Regs<At::S>& R) const {
+    at.seg(r, R.r);
+    if constexpr (NV) at.seg(nv, R.nv);
     else fill_regs(R.nv, 0.f);
-    load_seg<S, VEC>(term + o, t0, T, R.te);
+    at.seg(term, R.te);
     if constexpr (TRUNC) {
-      load_seg<S, VEC>(trunc + o, t0, T, R.tr);
-      boot_load<S, VEC, true>(boot, boot_mode, row, t0, T, R.bt, R.blast, r + o);
+      at.seg(trunc, R.tr);
+      boot_load<true>(at, boot, boot_mode, R.bt, R.blast, r);
     } else {
       fill_regs(R.tr, 0.f), fill_regs(R.bt, 0.f);
       R.blast = 0.f;
@@ -590,8 +884,9 @@ struct ReturnsOp {
       m[i].mul = in ? gl * nd : 1.f;
     }
   }
-  __device__ const E* row_carry_src(int64_t row, int T) const {
-    return boot_mode == kBootNone ? nullptr : boot_last(boot, boot_mode, row, T);
+  template <class At>
+  __device__ const E* row_carry_src(const At& at) const {
+    return boot_mode == kBootNone ? nullptr : boot_last(at, boot, boot_mode);
   }
 
   template <int S, int VEC, int SP = 0>
@@ -630,17 +925,17 @@ struct DoneGatedForwardOp {
     float x[S], d[S];
   };
 
-  template <int S, int VEC>
-  __device__ void load(int64_t row, int t0, int T, Regs<S>& R) const {
-    const int64_t o = row * (int64_t)T;
-    load_seg<S, VEC>(x + o, t0, T, R.x);
-    load_seg<S, VEC>(dones + o, t0, T, R.d);
+  template <class At>
+  __device__ void load(const At& at, Regs<At::S>& R) const {
+    at.seg(x, R.x);
+    at.seg(dones, R.d);
   }
   template <int S, int VEC>
   __device__ void prepare(Regs<S>&, int64_t, int, int) const {}
   template <int S>
   __device__ float export_last(const Regs<S>& R) const { return R.d[S - 1]; }
-  __device__ float halo_load(int64_t row, int t, int T) const { return to_f32(dones[row * (int64_t)T + t]); }
+  template <class At>
+  __device__ float halo_load(const At& at, int t, const Regs<At::S>&) const { return to_f32(dones[at.index(t)]); }
 
   template <int S, int VEC = kElementAligned>
   __device__ void coef(const Regs<S>& R, float dh, int64_t, int t0, int T, Affine (&m)[S]) const {
@@ -661,7 +956,8 @@ struct DoneGatedForwardOp {
       m[i].add = in ? R.x[i] : 0.f;
     }
   }
-  __device__ const E* row_carry_src(int64_t row, int) const { return seed ? seed + row : nullptr; }
+  template <class At>
+  __device__ const E* row_carry_src(const At& at) const { return seed ? seed + at.row : nullptr; }
 
   template <int S, int VEC, int SP = 0>
   __device__ void emit(const Regs<S>&, float, const float (&xs)[S], float, int64_t row, int t0,
@@ -692,11 +988,10 @@ struct AffineScanOp {
   struct Regs {
     float u[S], v[S];
   };
-  template <int S, int VEC>
-  __device__ void load(int64_t row, int t0, int T, Regs<S>& R) const {
-    const int64_t o = row * (int64_t)T;
-    load_seg<S, VEC>(u + o, t0, T, R.u);
-    load_seg<S, VEC>(v + o, t0, T, R.v);
+  template <class At>
+  __device__ void load(const At& at, Regs<At::S>& R) const {
+    at.seg(u, R.u);
+    at.seg(v, R.v);
   }
   template <int S, int VEC>
   __device__ void prepare(Regs<S>&, int64_t, int, int) const {}
@@ -709,7 +1004,8 @@ struct AffineScanOp {
       m[i].add = in ? R.u[i] : 0.f;
     }
   }
-  __device__ const E* row_carry_src(int64_t row, int) const { return carry ? carry + row : nullptr; }
+  template <class At>
+  __device__ const E* row_carry_src(const At& at) const { return carry ? carry + at.row : nullptr; }
   template <int S, int VEC, int SP = 0>
   __device__ void emit(const Regs<S>&, NoHalo, const float (&xs)[S], float, int64_t row, int t0,
                        int T) const {

@@ -38,6 +38,7 @@ int retrace_impl(const E* action_probs_target, const E* action_probs_behavior, c
   switch (A) {
     case 1: RLK_RETRACE(1)
     case 2: RLK_RETRACE(2)
+    case 3: RLK_RETRACE(3)
     case 4: RLK_RETRACE(4)
     default: RLK_RETRACE(0)
   }
