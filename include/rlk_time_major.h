@@ -1,0 +1,61 @@
+/*
+ * rlk_time_major.h -- calls on time-major arrays, between the PyTorch extension and
+ * librl_triton_amd.so (not part of the C ABI of rl_triton_amd.h).
+ *
+ * A call's [num_envs, seq_len] inputs are transposed views of [seq_len, num_envs] buffers:
+ * element (env, t) at env + t * step_stride of every array (Retrace's action rows at
+ * (env + t * step_stride) * num_actions).  One kernel reads them in place; the outputs are
+ * contiguous [num_envs, seq_len] arrays.  Results are those of the op's rl_triton_amd.h entry
+ * point on contiguous copies, up to the order of float32 sums; no workspace.
+ */
+#ifndef RLK_TIME_MAJOR_H
+#define RLK_TIME_MAJOR_H
+
+#include <stddef.h>
+#include <stdint.h>
+
+#ifdef __cplusplus
+extern "C" {
+#endif
+
+enum rlk_op {
+  RLK_OP_GAE,                /* in: rewards, values, terminateds, truncateds, mask */
+  RLK_OP_GAE_NORMALIZED,     /* the same; out: advantages, returns */
+  RLK_OP_VTRACE,             /* in: log_pi_target, log_pi_behavior, values, rewards,
+                                terminateds, truncateds; out: targets, advantages */
+  RLK_OP_RETRACE,            /* in: action_probs_target, action_probs_behavior, q_values,
+                                next_q_values_all, actions, rewards, terminateds, truncateds;
+                                out: targets, advantages */
+  RLK_OP_LAMBDA_RETURNS,     /* in: rewards, next_values, terminateds, truncateds */
+  RLK_OP_DISCOUNTED_RETURNS, /* in: rewards, terminateds, truncateds */
+  RLK_OP_FORWARD             /* traces and prefix sum; in: x, dones; bootstrap: seed_values */
+};
+
+typedef struct rlk_time_major_call {
+  int op;
+  int bf16;             /* 0: float32 arrays, 1: bfloat16 */
+  const void *in[8];    /* as listed above, NULL where absent */
+  const void *bootstrap;
+  int boot_mode;        /* RLK_BOOT_* (RLK_OP_FORWARD: ignored) */
+  int ends_at;          /* RLK_OP_FORWARD */
+  void *out[2];
+  int64_t num_envs, seq_len, step_stride, num_actions;
+  float gamma, lambda_; /* RLK_OP_FORWARD: gamma is the decay */
+  float rho_bar, c_bar, eps;
+  void *partials;       /* RLK_OP_GAE_NORMALIZED: rlk_time_major_partials_bytes bytes */
+  size_t partials_bytes;
+} rlk_time_major_call;
+
+/* 1 if calls of this shape are taken (rlk_time_major returns RLK_ERR_INVALID_ARGUMENT for
+ * others): rows of up to 2048 steps, and for Retrace (num_actions > 0) with more than four
+ * actions up to 512 steps or at least 1024 environments.  Other calls are faster through
+ * contiguous copies. */
+int rlk_time_major_takes(int64_t num_envs, int64_t seq_len, int64_t step_stride, int64_t num_actions);
+size_t rlk_time_major_partials_bytes(int64_t num_envs, int64_t seq_len);
+int rlk_time_major(const rlk_time_major_call *call, void *stream);
+
+#ifdef __cplusplus
+}
+#endif
+
+#endif /* RLK_TIME_MAJOR_H */

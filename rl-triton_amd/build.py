@@ -53,7 +53,7 @@ def sources() -> list[str]:
 
 def deps() -> list[str]:
     return sources() + sorted(glob.glob(os.path.join(CSRC, "*.hpp"))) + [
-        os.path.join(INCLUDE, "rl_triton_amd.h"), os.path.abspath(__file__)]
+        os.path.join(INCLUDE, "rl_triton_amd.h"), os.path.join(INCLUDE, "rlk_time_major.h"), os.path.abspath(__file__)]
 
 
 def up_to_date(target: str, inputs: list[str]) -> bool:
@@ -100,7 +100,7 @@ def build_ceiling(force: bool = True, verbose: bool = False) -> str:
 def build_ext(force: bool = True, verbose: bool = False) -> str:
     """_rlk_torch.so: a CPython extension module (no pybind11) linked against torch's
     libraries and against librl_triton_amd.so, found next to it at run time."""
-    inputs = [EXT_SRC, os.path.join(INCLUDE, "rl_triton_amd.h"), os.path.abspath(__file__), LIB]
+    inputs = [EXT_SRC, os.path.join(INCLUDE, "rl_triton_amd.h"), os.path.join(INCLUDE, "rlk_time_major.h"), os.path.abspath(__file__), LIB]
     if not force and up_to_date(EXT, inputs):
         return EXT
     import sysconfig

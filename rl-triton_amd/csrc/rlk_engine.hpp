@@ -409,9 +409,9 @@ struct RowAt {
   }
 };
 
-// ColumnAt: [T, E] in memory, steps ld elements apart; COLS environments side by side in a wave
+// ColumnAt: [T, E] in memory, steps ld elements apart; 16 environments side by side in a wave
 // (rlk_columns.hpp).  Steps beyond T read the last one.
-template <int S_, int COLS>
+template <int S_>
 struct ColumnAt {
   static constexpr int S = S_, kVec = kElementAligned;
   int64_t row;
@@ -432,8 +432,8 @@ struct ColumnAt {
 // Environments side by side in a wave (rows: one, of up to kWave lanes).
 template <class At>
 struct columns_of : std::integral_constant<int, kWave> {};
-template <int S, int COLS>
-struct columns_of<ColumnAt<S, COLS>> : std::integral_constant<int, COLS> {};
+template <int S>
+struct columns_of<ColumnAt<S>> : std::integral_constant<int, 16> {};
 
 // Address of boot(T-1) of the row (g_zero when there is no bootstrap).
 template <class At, class E>

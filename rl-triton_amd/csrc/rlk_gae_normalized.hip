@@ -1,28 +1,9 @@
 // rlk_gae_normalized.hip -- normalised GAE entry points (include/rl_triton_amd.h).
 #include "rlk_launch.hpp"
+#include "rlk_normalize.hpp"
 
 namespace rlk {
 namespace {
-
-// First launches of more workgroups than this have their partials summed by a tree of
-// reduce_partials_kernel levels (kReduceSlice triples into one per level) until at most
-// this many remain, which normalize_kernel's workgroups then each read.  The crossover,
-// measured on MI355X (float32, µs per call): 2048 triples read directly 24.1, through one
-// level 24.7 ([32768,128]); 4096 triples 44.9 directly, 42.5 through a level ([65536,128]).
-// Against every normalising workgroup reading every triple, the tree takes [2^20,128]
-// (65536 triples) from 761 to 630 µs and [16384,2048] from 167 to 139 µs.
-constexpr int64_t kDirectParts = 2048;
-
-// Triples of the partials buffer for a first launch of `nparts` workgroups: its own, then
-// each tree level's.
-int64_t partials_triples(int64_t nparts) {
-  int64_t total = nparts;
-  for (int64_t n = nparts; n > kDirectParts;) {
-    n = (n + kReduceSlice - 1) / kReduceSlice;
-    total += n;
-  }
-  return total;
-}
 
 // Partials of compute_gae_normalized: kStatWords doubles per workgroup of the first launch
 // and per tree level, for the larger of the two ops' grids (the masked op uses narrower
@@ -42,38 +23,12 @@ int normalized_launch(StatsOp op, E* advantages, int64_t num_envs, int64_t seq_l
                       float eps, void* workspace, size_t workspace_bytes, void* partials,
                       size_t partials_bytes, void* stream) {
   if (num_envs < 0 || seq_len < 0 || seq_len > (int64_t{1} << 30)) return RLK_ERR_INVALID_ARGUMENT;
-  double* parts = reinterpret_cast<double*>(partials);
   const int64_t nparts = call_blocks<StatsOp>(num_envs, seq_len);
-  if (parts == nullptr || (reinterpret_cast<uintptr_t>(parts) & 7u) != 0 ||
-      partials_bytes < (size_t)partials_triples(nparts) * kStatWords * sizeof(double) ||
-      nparts > 0x7fffffffLL)
-    return RLK_ERR_WORKSPACE;
-  op.partials = parts;
+  if (!partials_fit(partials, partials_bytes, nparts)) return RLK_ERR_WORKSPACE;
+  op.partials = reinterpret_cast<double*>(partials);
   const int st = launch(op, num_envs, seq_len, vec, workspace, workspace_bytes, stream);
   if (st != RLK_OK) return st;
-  hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-  int np = (int)nparts;
-  while (np > kDirectParts) {
-    const int next = (np + kReduceSlice - 1) / kReduceSlice;
-    double* up = parts + kStatWords * (int64_t)np;
-    void* rargs[] = {&parts, &np, &up};
-    if (hipLaunchKernel(reinterpret_cast<const void*>(&reduce_partials_kernel<kReduceNT>),
-                        dim3((unsigned)next), dim3(kReduceNT), rargs, 0, s) != hipSuccess)
-      return RLK_ERR_LAUNCH;
-    parts = up;
-    np = next;
-  }
-  constexpr int kNormNT = 256;
-  int64_t n = num_envs * seq_len;
-  const bool nvec = n % 4 == 0 && quad_aligned(advantages);
-  const int64_t units = nvec ? n / 4 : n;
-  int64_t grid = (units + kNormNT - 1) / kNormNT;
-  if (grid > 2048) grid = 2048;
-  void* args[] = {&advantages, &parts, &np, &n, &eps};
-  const void* kernel = nvec ? reinterpret_cast<const void*>(&normalize_kernel<kNormNT, true, E>)
-                            : reinterpret_cast<const void*>(&normalize_kernel<kNormNT, false, E>);
-  const hipError_t e = hipLaunchKernel(kernel, dim3((unsigned)grid), dim3(kNormNT), args, 0, s);
-  return e == hipSuccess ? RLK_OK : RLK_ERR_LAUNCH;
+  return normalize(advantages, op.partials, nparts, num_envs * seq_len, eps, reinterpret_cast<hipStream_t>(stream));
 }
 
 // mask == nullptr: every step counts (GaeStatsOp); otherwise the masked op

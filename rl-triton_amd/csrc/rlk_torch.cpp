@@ -3,7 +3,8 @@
 // Python module rl_triton._rlk_torch.  One function per estimator takes the public API's
 // arguments as they were passed.  When the call can go to the C ABI as it stands, the
 // function allocates the outputs, launches on torch's current stream and returns them.
-// That needs every tensor to be a contiguous tensor of the expected dtype (float32, or
+// That needs every tensor to be a contiguous tensor (or, for the public functions on rows of up
+// to 2048 steps, every one a transposed view of a [T, E] buffer) of the expected dtype (float32, or
 // bfloat16 throughout) and shape on the current GPU, RL_TRITON_CORRECTNESS_WARNINGS unset,
 // and, for rows long enough to need a look-back workspace, a stream that is not capturing
 // a graph (captured calls get buffers of their own on the Python path).  Any other call
@@ -33,6 +34,7 @@
 #include <utility>
 
 #include "rl_triton_amd.h"
+#include "rlk_time_major.h"
 
 namespace {
 
@@ -47,6 +49,11 @@ PyObject* decline() { Py_RETURN_NONE; }
 struct Call {
   c10::DeviceIndex dev = -1;
   int64_t E = 0, T = 0;
+  // Transposed views of [T, E] buffers (rollout buffers filled step by step) are taken too:
+  // every [E, T] tensor then has strides (1, ld) with one ld for the call, Retrace's [E, T, A]
+  // ones (A, ld * A, 1).  ld == 0: contiguous rows.
+  bool columns_ok = false;
+  int64_t ld = 0;
   at::ScalarType io = at::kFloat;  // the storage type of every float tensor of the call
   bool ok = true;
 
@@ -58,12 +65,14 @@ struct Call {
     if (!ok || !THPVariable_Check(o)) return fail();
     const at::Tensor& t = THPVariable_Unpack(o);
     io = t.scalar_type();
-    if (!t.is_cuda() || t.dim() != 2 || (io != at::kFloat && io != at::kBFloat16) ||
-        !t.is_contiguous())
-      return fail();
-    dev = t.get_device();
+    if (!t.is_cuda() || t.dim() != 2 || (io != at::kFloat && io != at::kBFloat16)) return fail();
     E = t.size(0);
     T = t.size(1);
+    if (!t.is_contiguous()) {
+      ld = t.stride(1);
+      if (!columns_ok || t.is_neg() || t.stride(0) != 1 || !rlk_time_major_takes(E, T, ld, 0)) return fail();
+    }
+    dev = t.get_device();
     if (dev != c10::hip::current_device()) return fail();
     return &t;
   }
@@ -74,8 +83,15 @@ struct Call {
     if (st == at::ScalarType::Undefined) st = io;
     if (!ok || !THPVariable_Check(o)) return fail();
     const at::Tensor& t = THPVariable_Unpack(o);
-    if (!t.is_cuda() || t.get_device() != dev || t.scalar_type() != st || !t.is_contiguous())
-      return fail();
+    if (!t.is_cuda() || t.get_device() != dev || t.scalar_type() != st) return fail();
+    if (ld == 0 || kind == 1) {
+      if (!t.is_contiguous()) return fail();
+    } else {
+      const int64_t a = kind == 3 ? A : 1;
+      if (t.is_neg() || t.dim() != kind || t.stride(0) != a || t.stride(1) != ld * a ||
+          (kind == 3 && A > 1 && t.stride(2) != 1))
+        return fail();
+    }
     const bool shape_ok = kind == 1   ? (t.dim() == 1 && t.size(0) == E)
                         : kind == 2   ? (t.dim() == 2 && t.size(0) == E && t.size(1) == T)
                                       : (t.dim() == 3 && t.size(0) == E && t.size(1) == T &&
@@ -109,6 +125,20 @@ struct Call {
     return at::Tensor(at::detail::empty_cuda({E, T}, like.scalar_type(), like.device(), std::nullopt));
   }
 };
+
+// A call on time-major arrays (c.ld > 0): the op's inputs in rlk_time_major.h's order, its
+// scalars by name.  `tensors`: n of them, nullptr where absent.
+rlk_time_major_call time_major(const Call& c, int op, const at::Tensor* const* tensors, int n,
+                               const at::Tensor* boot, int boot_mode) {
+  rlk_time_major_call t = {};
+  t.op = op;
+  t.bf16 = c.bf16() ? 1 : 0;
+  for (int i = 0; i < n; ++i) t.in[i] = tensors[i] ? tensors[i]->data_ptr() : nullptr;
+  t.bootstrap = boot ? boot->data_ptr() : nullptr;
+  t.boot_mode = boot_mode;
+  t.num_envs = c.E, t.seq_len = c.T, t.step_stride = c.ld;
+  return t;
+}
 
 // Look-back workspaces of the calls this module launches, one per (device, stream):
 // zero-filled when allocated (on that stream), grown by doubling, and left ready by every
@@ -249,11 +279,13 @@ bool nargs_is(Py_ssize_t n, Py_ssize_t want, const char* name) {
 
 // gae(rewards, values, terminateds, truncateds, gamma, lambda_, bootstrap_values, last_value,
 //     mask)
+template <bool COLUMNS>
 PyObject* op_gae(PyObject* const* a, Py_ssize_t n) {
   if (!nargs_is(n, 9, "gae")) return nullptr;
   prefetch_tensors(a, n);
   if (correctness_warnings()) return decline();
   Call c;
+  c.columns_ok = COLUMNS;
   const at::Tensor* r = c.lead(a[0]);
   const at::Tensor* v = c.need(a[1]);
   const at::Tensor* te = c.need(a[2]);
@@ -266,6 +298,14 @@ PyObject* op_gae(PyObject* const* a, Py_ssize_t n) {
   const at::Tensor* mask = c.opt(a[8]);
   if (!c.ok) return decline();
   const int mode = has_lv ? RLK_BOOT_ROW : has_bv ? RLK_BOOT_FULL : RLK_BOOT_NONE;
+  if (c.ld > 0) {
+    const at::Tensor* in[] = {r, v, te, tr, mask};
+    rlk_time_major_call t = time_major(c, RLK_OP_GAE, in, 5, boot, mode);
+    t.gamma = gamma, t.lambda_ = lam;
+    at::Tensor out = c.output(*r);
+    t.out[0] = out.data_ptr();
+    return finish(rlk_time_major(&t, c.stream()), "rlk_time_major", THPVariable_Wrap(std::move(out)));
+  }
   const Workspace ws = workspace(c, *r);
   if (!ws.ok) return decline();
   at::Tensor out = c.output(*r);
@@ -283,11 +323,13 @@ PyObject* op_gae(PyObject* const* a, Py_ssize_t n) {
 
 // gae_normalized(rewards, values, terminateds, truncateds, gamma, lambda_, bootstrap_values,
 //                last_value, eps, mask) -> (advantages, returns)
+template <bool COLUMNS>
 PyObject* op_gae_normalized(PyObject* const* a, Py_ssize_t n) {
   if (!nargs_is(n, 10, "gae_normalized")) return nullptr;
   prefetch_tensors(a, n);
   if (correctness_warnings()) return decline();
   Call c;
+  c.columns_ok = COLUMNS;
   const at::Tensor* r = c.lead(a[0]);
   const at::Tensor* v = c.need(a[1]);
   const at::Tensor* te = c.need(a[2]);
@@ -300,6 +342,16 @@ PyObject* op_gae_normalized(PyObject* const* a, Py_ssize_t n) {
   const at::Tensor* mask = c.opt(a[9]);
   if (!c.ok) return decline();
   const int mode = has_lv ? RLK_BOOT_ROW : has_bv ? RLK_BOOT_FULL : RLK_BOOT_NONE;
+  if (c.ld > 0) {
+    const at::Tensor* in[] = {r, v, te, tr, mask};
+    rlk_time_major_call t = time_major(c, RLK_OP_GAE_NORMALIZED, in, 5, boot, mode);
+    t.gamma = gamma, t.lambda_ = lam, t.eps = eps;
+    at::Tensor adv = c.output(*r), ret = c.output(*r);
+    t.partials_bytes = rlk_time_major_partials_bytes(c.E, c.T);
+    at::Tensor parts = at::empty({(int64_t)t.partials_bytes}, r->options().dtype(at::kByte));
+    t.out[0] = adv.data_ptr(), t.out[1] = ret.data_ptr(), t.partials = parts.data_ptr();
+    return finish(rlk_time_major(&t, c.stream()), "rlk_time_major", pair(adv, ret));
+  }
   const Workspace ws = workspace(c, *r);
   if (!ws.ok) return decline();
   at::Tensor adv = c.output(*r), ret = c.output(*r);
@@ -321,11 +373,13 @@ PyObject* op_gae_normalized(PyObject* const* a, Py_ssize_t n) {
 
 // vtrace(log_pi_target, log_pi_behavior, values, rewards, terminateds, truncateds, gamma,
 //        rho_bar, c_bar, bootstrap_values, last_value)
+template <bool COLUMNS>
 PyObject* op_vtrace(PyObject* const* a, Py_ssize_t n) {
   if (!nargs_is(n, 11, "vtrace")) return nullptr;
   prefetch_tensors(a, n);
   if (correctness_warnings()) return decline();
   Call c;
+  c.columns_ok = COLUMNS;
   const at::Tensor* r = c.lead(a[3]);
   const at::Tensor* lpt = c.need(a[0]);
   const at::Tensor* lpb = c.need(a[1]);
@@ -338,6 +392,14 @@ PyObject* op_vtrace(PyObject* const* a, Py_ssize_t n) {
   const at::Tensor* boot = has_lv ? c.need(a[10], 1) : c.opt(a[9]);
   if (!c.ok) return decline();
   const int mode = has_lv ? RLK_BOOT_ROW : has_bv ? RLK_BOOT_FULL : RLK_BOOT_NONE;
+  if (c.ld > 0) {
+    const at::Tensor* in[] = {lpt, lpb, v, r, te, tr};
+    rlk_time_major_call t = time_major(c, RLK_OP_VTRACE, in, 6, boot, mode);
+    t.gamma = gamma, t.rho_bar = rho_bar, t.c_bar = c_bar;
+    at::Tensor tg = c.output(*r), adv = c.output(*r);
+    t.out[0] = tg.data_ptr(), t.out[1] = adv.data_ptr();
+    return finish(rlk_time_major(&t, c.stream()), "rlk_time_major", pair(tg, adv));
+  }
   const Workspace ws = workspace(c, *r);
   if (!ws.ok) return decline();
   at::Tensor tg = c.output(*r), adv = c.output(*r);
@@ -352,11 +414,13 @@ PyObject* op_vtrace(PyObject* const* a, Py_ssize_t n) {
 
 // retrace(action_probs_target, action_probs_behavior, q_values, next_q_values_all, actions,
 //         rewards, terminateds, truncateds, gamma, lambda_, c_bar, rho_bar)
+template <bool COLUMNS>
 PyObject* op_retrace(PyObject* const* a, Py_ssize_t n) {
   if (!nargs_is(n, 12, "retrace")) return nullptr;
   prefetch_tensors(a, n);
   if (correctness_warnings()) return decline();
   Call c;
+  c.columns_ok = COLUMNS;
   const at::Tensor* r = c.lead(a[5]);
   int64_t A = 0;
   if (c.ok && THPVariable_Check(a[0])) {
@@ -374,6 +438,15 @@ PyObject* op_retrace(PyObject* const* a, Py_ssize_t n) {
   const float gamma = c.scalar(a[8]), lam = c.scalar(a[9]), c_bar = c.scalar(a[10]),
               rho_bar = c.scalar(a[11]);
   if (!c.ok) return decline();
+  if (c.ld > 0) {
+    if (!rlk_time_major_takes(c.E, c.T, c.ld, A)) return decline();
+    const at::Tensor* in[] = {pi, mu, q, nq, act, r, te, tr};
+    rlk_time_major_call t = time_major(c, RLK_OP_RETRACE, in, 8, nullptr, RLK_BOOT_NONE);
+    t.num_actions = A, t.gamma = gamma, t.lambda_ = lam, t.rho_bar = rho_bar, t.c_bar = c_bar;
+    at::Tensor tg = c.output(*r), adv = c.output(*r);
+    t.out[0] = tg.data_ptr(), t.out[1] = adv.data_ptr();
+    return finish(rlk_time_major(&t, c.stream()), "rlk_time_major", pair(tg, adv));
+  }
   const Workspace ws = workspace(c, *r);
   if (!ws.ok) return decline();
   at::Tensor tg = c.output(*r), adv = c.output(*r);
@@ -388,11 +461,13 @@ PyObject* op_retrace(PyObject* const* a, Py_ssize_t n) {
 }
 
 // lambda_returns(rewards, next_values, terminateds, truncateds, gamma, lambda_, bootstrap_values)
+template <bool COLUMNS>
 PyObject* op_lambda_returns(PyObject* const* a, Py_ssize_t n) {
   if (!nargs_is(n, 7, "lambda_returns")) return nullptr;
   prefetch_tensors(a, n);
   if (correctness_warnings()) return decline();
   Call c;
+  c.columns_ok = COLUMNS;
   const at::Tensor* r = c.lead(a[0]);
   const at::Tensor* nv = c.need(a[1]);
   const at::Tensor* te = c.need(a[2]);
@@ -400,6 +475,14 @@ PyObject* op_lambda_returns(PyObject* const* a, Py_ssize_t n) {
   const float gamma = c.scalar(a[4]), lam = c.scalar(a[5]);
   const at::Tensor* boot = c.opt(a[6]);
   if (!c.ok) return decline();
+  if (c.ld > 0) {
+    const at::Tensor* in[] = {r, nv, te, tr};
+    rlk_time_major_call t = time_major(c, RLK_OP_LAMBDA_RETURNS, in, 4, boot, boot ? RLK_BOOT_FULL : RLK_BOOT_NONE);
+    t.gamma = gamma, t.lambda_ = lam;
+    at::Tensor out = c.output(*r);
+    t.out[0] = out.data_ptr();
+    return finish(rlk_time_major(&t, c.stream()), "rlk_time_major", THPVariable_Wrap(std::move(out)));
+  }
   const Workspace ws = workspace(c, *r);
   if (!ws.ok) return decline();
   at::Tensor out = c.output(*r);
@@ -413,17 +496,27 @@ PyObject* op_lambda_returns(PyObject* const* a, Py_ssize_t n) {
 }
 
 // discounted_returns(rewards, terminateds, truncateds, gamma, bootstrap_values)
+template <bool COLUMNS>
 PyObject* op_discounted_returns(PyObject* const* a, Py_ssize_t n) {
   if (!nargs_is(n, 5, "discounted_returns")) return nullptr;
   prefetch_tensors(a, n);
   if (correctness_warnings()) return decline();
   Call c;
+  c.columns_ok = COLUMNS;
   const at::Tensor* r = c.lead(a[0]);
   const at::Tensor* te = c.need(a[1]);
   const at::Tensor* tr = c.opt(a[2]);
   const float gamma = c.scalar(a[3]);
   const at::Tensor* boot = c.opt(a[4]);
   if (!c.ok) return decline();
+  if (c.ld > 0) {
+    const at::Tensor* in[] = {r, te, tr};
+    rlk_time_major_call t = time_major(c, RLK_OP_DISCOUNTED_RETURNS, in, 3, boot, boot ? RLK_BOOT_FULL : RLK_BOOT_NONE);
+    t.gamma = gamma;
+    at::Tensor out = c.output(*r);
+    t.out[0] = out.data_ptr();
+    return finish(rlk_time_major(&t, c.stream()), "rlk_time_major", THPVariable_Wrap(std::move(out)));
+  }
   const Workspace ws = workspace(c, *r);
   if (!ws.ok) return decline();
   at::Tensor out = c.output(*r);
@@ -437,16 +530,26 @@ PyObject* op_discounted_returns(PyObject* const* a, Py_ssize_t n) {
 }
 
 // eligibility_traces(gradients, dones, gamma, lambda_, seed_values)
+template <bool COLUMNS>
 PyObject* op_eligibility_traces(PyObject* const* a, Py_ssize_t n) {
   if (!nargs_is(n, 5, "eligibility_traces")) return nullptr;
   prefetch_tensors(a, n);
   if (correctness_warnings()) return decline();
   Call c;
+  c.columns_ok = COLUMNS;
   const at::Tensor* g = c.lead(a[0]);
   const at::Tensor* d = c.need(a[1]);
   const float gamma = c.scalar(a[2]), lam = c.scalar(a[3]);
   const at::Tensor* seed = c.opt(a[4], 1);
   if (!c.ok) return decline();
+  if (c.ld > 0) {
+    const at::Tensor* in[] = {g, d};
+    rlk_time_major_call t = time_major(c, RLK_OP_FORWARD, in, 2, seed, RLK_BOOT_NONE);
+    t.gamma = gamma * lam, t.ends_at = 1;
+    at::Tensor out = c.output(*g);
+    t.out[0] = out.data_ptr();
+    return finish(rlk_time_major(&t, c.stream()), "rlk_time_major", THPVariable_Wrap(std::move(out)));
+  }
   const Workspace ws = workspace(c, *g);
   if (!ws.ok) return decline();
   at::Tensor out = c.output(*g);
@@ -459,15 +562,25 @@ PyObject* op_eligibility_traces(PyObject* const* a, Py_ssize_t n) {
 }
 
 // prefix_sum(inputs, dones, seed_values, ends_at)   (ends_at: the boundary, already checked)
+template <bool COLUMNS>
 PyObject* op_prefix_sum(PyObject* const* a, Py_ssize_t n) {
   if (!nargs_is(n, 4, "prefix_sum")) return nullptr;
   prefetch_tensors(a, n);
   if (correctness_warnings()) return decline();
   Call c;
+  c.columns_ok = COLUMNS;
   const at::Tensor* x = c.lead(a[0]);
   const at::Tensor* d = c.need(a[1]);
   const at::Tensor* seed = c.opt(a[2], 1);
   if (!c.ok || !PyBool_Check(a[3])) return decline();
+  if (c.ld > 0) {
+    const at::Tensor* in[] = {x, d};
+    rlk_time_major_call t = time_major(c, RLK_OP_FORWARD, in, 2, seed, RLK_BOOT_NONE);
+    t.gamma = 1.f, t.ends_at = a[3] == Py_True ? 1 : 0;
+    at::Tensor out = c.output(*x);
+    t.out[0] = out.data_ptr();
+    return finish(rlk_time_major(&t, c.stream()), "rlk_time_major", THPVariable_Wrap(std::move(out)));
+  }
   const Workspace ws = workspace(c, *x);
   if (!ws.ok) return decline();
   at::Tensor out = c.output(*x);
@@ -531,7 +644,7 @@ PyObject* op_prefix_sum_api(PyObject* const* a, Py_ssize_t n) {
   else if (PyUnicode_CompareWithASCIIString(a[3], "starts_at") == 0) ends_at = Py_False;
   else return decline();  // the Python path raises its ValueError
   PyObject* b[4] = {a[0], a[1], a[2], ends_at};
-  return op_prefix_sum(b, 4);
+  return op_prefix_sum<true>(b, 4);
 }
 
 constexpr int kMaxParams = 16;
@@ -607,21 +720,23 @@ PyGetSetDef kEntryGetSet[] = {
 
 PyTypeObject EntryType = {PyVarObject_HEAD_INIT(nullptr, 0)};
 
+// The module's own functions take contiguous rows only, the public entries (kOps) transposed
+// views too.
 #define RLK_METHOD(name) \
-  { #name, (PyCFunction)(void (*)(void))guarded<op_##name>, METH_FASTCALL, nullptr }
+  { #name, (PyCFunction)(void (*)(void))guarded<op_##name<false>>, METH_FASTCALL, nullptr }
 
 struct OpName {
   const char* name;
   FastOp op;
 };
 const OpName kOps[] = {
-    {"gae", guarded<op_gae>},
-    {"gae_normalized", guarded<op_gae_normalized>},
-    {"vtrace", guarded<op_vtrace>},
-    {"retrace", guarded<op_retrace>},
-    {"lambda_returns", guarded<op_lambda_returns>},
-    {"discounted_returns", guarded<op_discounted_returns>},
-    {"eligibility_traces", guarded<op_eligibility_traces>},
+    {"gae", guarded<op_gae<true>>},
+    {"gae_normalized", guarded<op_gae_normalized<true>>},
+    {"vtrace", guarded<op_vtrace<true>>},
+    {"retrace", guarded<op_retrace<true>>},
+    {"lambda_returns", guarded<op_lambda_returns<true>>},
+    {"discounted_returns", guarded<op_discounted_returns<true>>},
+    {"eligibility_traces", guarded<op_eligibility_traces<true>>},
     {"prefix_sum", guarded<op_prefix_sum_api>},
 };
 
@@ -716,7 +831,7 @@ PyMethodDef kMethods[] = {
     RLK_METHOD(discounted_returns),
     RLK_METHOD(eligibility_traces),
     RLK_METHOD(prefix_sum),
-    RLK_METHOD(affine_scan),
+    {"affine_scan", (PyCFunction)(void (*)(void))guarded<op_affine_scan>, METH_FASTCALL, nullptr},
     {nullptr, nullptr, 0, nullptr}};
 
 PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "_rlk_torch",
