@@ -111,9 +111,9 @@ int rlk_debug_lookback(int give_up_polls, int fallback_polls);
  * their outputs non-temporally or write-through, chosen per launch by the call's shape and
  * storage type (a speed choice; the bits stored are the same).  policy 0 or 1 forces
  * non-temporal or write-through stores, process-wide, for the calls launched after it,
- * wherever the launch is built with that policy (bfloat16 outputs and the 1025..2048-step
- * strided rows are write-through only; float32 V-trace and Retrace long rows non-temporal
- * only); -1 restores the rule.  Returns RLK_OK, or RLK_ERR_INVALID_ARGUMENT for another
+ * wherever the launch is built with that policy (bfloat16 outputs, and rows of more than
+ * 1024 steps that one workgroup holds, are write-through only; float32 V-trace and Retrace
+ * rows split into tiles non-temporal only); -1 restores the rule.  Returns RLK_OK, or RLK_ERR_INVALID_ARGUMENT for another
  * value. */
 int rlk_debug_store_policy(int policy);
 

@@ -1267,14 +1267,19 @@ __device__ __forceinline__ SkipAffine lane_bcast(SkipAffine m, int l) {
 
 constexpr int kSeg = 4;  // steps per segment of the long-row path
 
-// Rows of 1025..2048 steps, one per workgroup, with the long-row tile layout: NT threads
-// hold Q segments of 4 steps each, strided by the wave (segment q of lane l at step
-// (q*64 + l)*4 of the wave's chunk), so every vector access of a wave covers 1 KB.  Against
-// one segment per thread (rows_kernel with NT = 512) a row has half the waves, so its wave
-// maps chain through LDS in at most NW - 1 = 3 applies instead of 7.  Launch: grid = E.
+// One row per workgroup with the long-row tile layout: the workgroup's waves (blockDim.x / 64 of
+// them, at most NT / 64) hold Q segments of 4 steps per thread, strided by the wave (segment q of
+// lane l at step (q*64 + l)*4 of the wave's chunk), so every vector access of a wave covers 1 KB.
+// Two uses:
+//   * rows of 1025..2048 steps, 256 threads of Q = 2: against one segment per thread
+//     (rows_kernel with NT = 512) a row has half the waves, so its wave maps chain through LDS
+//     in at most 3 applies instead of 7;
+//   * longer rows of calls with a workgroup for every CU (whole_row in rlk_launch.hpp), as many
+//     waves as the row needs.
+// Launch: grid = E.
 template <class Op, int NT, int Q, int VEC, int SP = 0>
 __global__ __launch_bounds__(NT) void rows_strided_kernel(const Op op, int64_t E, int T, int) {
-  static_assert(VEC != kPhased, "phased access is for long rows");
+  static_assert(VEC != kPhased, "phased access is for rows split into tiles");
   constexpr bool FWD = Op::kForward;
   constexpr int NW = NT / kWave;
   constexpr int S = 4;
@@ -1289,9 +1294,10 @@ __global__ __launch_bounds__(NT) void rows_strided_kernel(const Op op, int64_t E
   const int tid = threadIdx.x;
   const int lane = __lane_id();
   const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+  const int nw = NW <= 4 ? NW : (int)(blockDim.x / kWave);
   const int64_t row = blockIdx.x;
   // lane space -> time: this wave's chunk, and the first step of segment row r
-  const int wbase = (FWD ? wave : NW - 1 - wave) * WSTEPS;
+  const int wbase = (FWD ? wave : nw - 1 - wave) * WSTEPS;
   const int lt = FWD ? lane : kWave - 1 - lane;
   auto seg_t0 = [&](int r) { return wbase + ((FWD ? r : Q - 1 - r) * kWave + lt) * S; };
   auto seg_at = [&](int r) { return RowAt<S, VEC>{row, seg_t0(r), T}; };
@@ -1335,7 +1341,14 @@ __global__ __launch_bounds__(NT) void rows_strided_kernel(const Op op, int64_t E
   if (lane == 0) s_map[wave] = wm;
   __syncthreads();
   // state entering this wave's chunk, then each segment row, then each lane
-  for (int v = 0; v < wave; ++v) carry = s_map[v].apply(carry);
+  if constexpr (NW <= 4) {
+    for (int v = 0; v < wave; ++v) carry = s_map[v].apply(carry);
+  } else if (wave > 0) {
+    // the waves before this one by a lane scan: applied one after another, each read waited for,
+    // sixteen take 0.9 us
+    Map pm = lane < wave ? s_map[lane] : Map::identity();
+    carry = lane_bcast(lane_scan(pm, NW), NW - 1).apply(carry);
+  }
   Stats st;
 #pragma unroll
   for (int r = 0; r < Q; ++r) {
@@ -1347,7 +1360,7 @@ __global__ __launch_bounds__(NT) void rows_strided_kernel(const Op op, int64_t E
     op.template emit<S, VEC, SP>(R[r], h[r], xs, x_in, row, seg_t0(r), T);
     if constexpr (Op::kBlockStats) op.template stats<S>(R[r], xs, seg_t0(r), T, st);
   }
-  if constexpr (Op::kBlockStats) block_stats<NT>(st, op.partials);
+  if constexpr (Op::kBlockStats) block_stats<NT>(st, op.partials, nw);
 }
 
 

@@ -262,10 +262,50 @@ bool step_per_thread(int64_t E, int64_t T) {
   return T <= kNTWide && E * T <= 8 * kWave * (int64_t)device_cus();  // 8 waves per CU
 }
 
-// Workgroups of the launch that launch() makes for Op at [E, T] (E, T > 0).
+// Rows of more than 2048 steps that one workgroup holds whole (rows_strided_kernel, as many waves
+// as the row needs): no look-back, no padding to a tile, few enough registers that two or more
+// workgroups share a CU (Q segments of 4 steps per thread: up to 1024 * 4 * Q steps).  Against
+// the look-back's tiles, on MI355X (us):
+//   * up to 8192 steps (Q = 1, 2) faster at every count of rows: GAE [4,2500] by 1.46x, [64,2049]
+//     4.34 -> 2.73, [512,5000] 12.2 -> 11.2, masked GAE [512,6000] 14.6 -> 10.6, [2000,5000]
+//     49.1 -> 34.1, V-trace [512,5000] 18.2 -> 13.3, bfloat16 [512,6000] 15.7 -> 9.3, TD(lambda)
+//     [2000,2049] 15.7 -> 11.1, prefix sum [2000,2049] 14.7 -> 9.2, [256,8192] 5.4 -> 4.6;
+//   * up to 16384 steps (Q = 4) with a row for every other CU: masked GAE [256,12000] 1.47x,
+//     V-trace 1.40x, GAE [512,10000] 1.11x; fewer rows leave CUs idle that tiles use (GAE
+//     [64,16384] 0.75x).  Element-aligned GAE and V-trace keep the phased tiles there ([512,15001]
+//     0.96x, 0.98x).
+// Retrace's action blocks fill the registers at Q = 2: rows above 4096 steps take it from a row
+// per CU on (A = 4 [16,8000] 0.84x, [512,7001] 1.01x, [256,5001] 1.36x).
+constexpr int kWholeRowThreads = 1024;
+enum class WholeRow { kNever, kTwoSegments, kFourSegments, kFourSegmentsAligned };
 template <class Op>
-int64_t launch_grid(int64_t E, int64_t T) {
+struct whole_row : std::integral_constant<WholeRow, WholeRow::kFourSegments> {};
+template <bool TRUNC, class E>
+struct whole_row<GaeOp<TRUNC, E>> : std::integral_constant<WholeRow, WholeRow::kFourSegmentsAligned> {};
+template <bool TRUNC, class E>
+struct whole_row<VtraceOp<TRUNC, E>> : std::integral_constant<WholeRow, WholeRow::kFourSegmentsAligned> {};
+template <int NA, bool TRUNC, class E>
+struct whole_row<RetraceOp<NA, TRUNC, E>>
+    : std::integral_constant<WholeRow, NA == 0 ? WholeRow::kNever : WholeRow::kTwoSegments> {};
+
+// Segments per thread of such a call, 0 for others.
+template <class Op>
+int whole_row_segments(int64_t E, int64_t T, bool vec) {
+  constexpr WholeRow k = whole_row<Op>::value;
+  constexpr int64_t steps = kWholeRowThreads * kSeg;
+  if (k == WholeRow::kNever || T <= kShortMaxT || T > 4 * steps) return 0;
+  if (T <= steps) return 1;
+  if (T <= 2 * steps) return k != WholeRow::kTwoSegments || E >= device_cus() ? 2 : 0;
+  if (k == WholeRow::kTwoSegments || 2 * E < device_cus()) return 0;
+  return vec || k != WholeRow::kFourSegmentsAligned ? 4 : 0;
+}
+
+// Workgroups of the launch that launch() makes for Op at [E, T] (E, T > 0).  (The grid of the
+// statistics ops, whose callers count workgroups, does not depend on vec.)
+template <class Op>
+int64_t launch_grid(int64_t E, int64_t T, bool vec = true) {
   if (T > kShortMaxT) {
+    if (whole_row_segments<Op>(E, T, vec) > 0) return E;
     const LongShape sh = long_shape<Op>(E, T);
     return chain_grid(E, T, sh.threads, sh.segments);
   }
@@ -325,14 +365,25 @@ struct strided_rows<VtraceOp<TRUNC, E>> : std::false_type {};
 template <int NA, bool TRUNC, class E>
 struct strided_rows<RetraceOp<NA, TRUNC, E>> : std::false_type {};
 
-template <class Op, int SP>
-hipError_t launch_strided(const Op& op, int64_t E, int T, hipStream_t stream) {
-  static_assert(kStridedThreads * kSeg * kStridedSegments == kShortMaxT, "one row per workgroup");
-  if (E * kStridedThreads > 0xffffffffLL) return hipErrorInvalidValue;  // launch() splits such calls
+// One row per workgroup of `threads` (at most NT), Q segments of 4 steps per thread.
+template <class Op, int NT, int Q, int VEC>
+hipError_t launch_strided(const Op& op, int64_t E, int T, int threads, hipStream_t stream) {
+  if (E * threads > 0xffffffffLL) return hipErrorInvalidValue;  // launch() splits such calls
   int unused = 0;
   void* args[] = {const_cast<Op*>(&op), &E, &T, &unused};
-  return hipLaunchKernel(reinterpret_cast<const void*>(&rows_strided_kernel<Op, kStridedThreads, kStridedSegments, kAligned, SP>),
-                         dim3((unsigned)E), dim3(kStridedThreads), args, dynamic_lds(op, kStridedThreads), stream);
+  return hipLaunchKernel(reinterpret_cast<const void*>(&rows_strided_kernel<Op, NT, Q, VEC, 1>),
+                         dim3((unsigned)E), dim3(threads), args, 0, stream);
+}
+
+template <class Op, int VEC>
+hipError_t launch_whole_row(const Op& op, int64_t E, int T, int segments, hipStream_t stream) {
+  const int wave_steps = kWave * kSeg * segments;
+  const int threads = kWave * ((T + wave_steps - 1) / wave_steps);
+  if (segments == 1) return launch_strided<Op, kWholeRowThreads, 1, VEC>(op, E, T, threads, stream);
+  if constexpr (whole_row<Op>::value != WholeRow::kTwoSegments) {
+    if (segments == 4) return launch_strided<Op, kWholeRowThreads, 4, VEC>(op, E, T, threads, stream);
+  }
+  return launch_strided<Op, kWholeRowThreads, 2, VEC>(op, E, T, threads, stream);
 }
 
 // Look-back poll budgets (rlk_debug_lookback): polls before a wait gives up (~1 s), and
@@ -414,7 +465,9 @@ hipError_t launch_long(const Op& op, int64_t E, int T, uint64_t* ws, hipStream_t
 //     V-trace and Retrace (discounted returns [16,131072] 8.00 -> 7.86, prefix sum
 //     [16,131072] 7.66 -> 7.49, TD(lambda) [8,262144] 8.92 -> 8.79); nt with more tiles
 //     (discounted [64,40000] 8.99 against 9.58) and for V-trace ([16,131072] 12.40 against
-//     12.70, [256,8192] 11.46 against 12.15).
+//     12.70);
+//   * rows held whole by a workgroup (rows_strided_kernel): sc1, 2-15% (GAE [256,2500] 3.63
+//     against 4.19, V-trace [512,4096] 10.2 against 10.8; equal at 2049 steps).
 // Plain stores were never the fastest by more than 3% and lost up to 13% elsewhere.  The
 // policy is a kernel template argument (SP), so a non-temporal instance is the same code
 // as before write-through stores existed.
@@ -435,15 +488,15 @@ struct long_rows_write_through<VtraceOp<TRUNC, E>> : std::false_type {};
 template <int NA, bool TRUNC, class E>
 struct long_rows_write_through<RetraceOp<NA, TRUNC, E>> : std::false_type {};
 
-enum class Kernel { kRows, kStrided, kChain };
-// The policies a kernel can be launched with for an op: bfloat16 outputs and the strided
-// rows kernel always write through, float32 V-trace and Retrace long rows never; only the
-// policies listed here are instantiated.
+enum class Kernel { kRows, kChain };
+// The policies a kernel can be launched with for an op: bfloat16 outputs always write through
+// (as rows_strided_kernel does), float32 V-trace and Retrace long rows never; only the policies
+// listed here are instantiated.
 template <class Op, Kernel K>
 struct store_policies {
   static constexpr bool kBf16 = std::is_same<typename Op::Elem, bf16>::value;
   static constexpr bool kWriteThrough = kBf16 || (K != Kernel::kChain && !one_form<Op>::value) || long_rows_write_through<Op>::value;
-  static constexpr bool kNonTemporal = !kBf16 && K != Kernel::kStrided;
+  static constexpr bool kNonTemporal = !kBf16;
   static_assert(kWriteThrough || kNonTemporal, "some store policy");
 };
 template <class Op, Kernel K>
@@ -566,16 +619,16 @@ void skip_rows(AffineScanOp<FWD, E>& op, int64_t r0, int64_t T) {
 // (a multiple of 512 where that is at least 512: whole workgroups of every short-row shape)
 // whose launch stays within kMaxLaunchBlocks.
 template <class Op>
-int64_t rows_per_launch(int64_t E, int64_t T) {
-  const int64_t g = launch_grid<Op>(E, T);
+int64_t rows_per_launch(int64_t E, int64_t T, bool vec = true) {
+  const int64_t g = launch_grid<Op>(E, T, vec);
   if (g <= kMaxLaunchBlocks) return E;
   int64_t n = (int64_t)((double)E * (double)kMaxLaunchBlocks / (double)g);  // grid ~ rows
   n = n < 1 ? 1 : n > E ? E : n;
   for (const int64_t unit : {int64_t{512}, int64_t{1}}) {
     if (n < unit) continue;
     int64_t m = n / unit * unit;
-    while (m > unit && launch_grid<Op>(m, T) > kMaxLaunchBlocks) m -= unit;
-    if (launch_grid<Op>(m, T) <= kMaxLaunchBlocks) return m;
+    while (m > unit && launch_grid<Op>(m, T, vec) > kMaxLaunchBlocks) m -= unit;
+    if (launch_grid<Op>(m, T, vec) <= kMaxLaunchBlocks) return m;
   }
   return 1;  // one row of at most 2^30 steps is at most 2^18 tiles
 }
@@ -599,7 +652,7 @@ int launch(const Op& op, int64_t E, int64_t T, bool vec, void* workspace, size_t
            void* stream, int phase0 = -1) {
   if (E < 0 || T < 0 || T > (int64_t{1} << 30)) return RLK_ERR_INVALID_ARGUMENT;
   if (E == 0 || T == 0) return RLK_OK;
-  const int64_t rows = rows_per_launch<Op>(E, T);
+  const int64_t rows = rows_per_launch<Op>(E, T, vec);
   if (rows < E) {
     int64_t blocks = 0;  // the statistics ops' partials of the ranges before this one
     for (int64_t r0 = 0; r0 < E; r0 += rows) {
@@ -621,6 +674,14 @@ int launch(const Op& op, int64_t E, int64_t T, bool vec, void* workspace, size_t
     uint64_t* ws = reinterpret_cast<uint64_t*>(workspace);
     if (ws == nullptr || workspace_bytes_given < workspace_bytes(E, T) || !aligned16(ws))
       return RLK_ERR_WORKSPACE;
+    if constexpr (whole_row<Op>::value != WholeRow::kNever) {
+      const int segments = whole_row_segments<Op>(E, T, vec);
+      if (segments > 0) {
+        e = vec ? launch_whole_row<Op, kAligned>(op, E, Ti, segments, s)
+                : launch_whole_row<Op, kElementAligned>(op, E, Ti, segments, s);
+        return e == hipSuccess ? RLK_OK : RLK_ERR_LAUNCH;
+      }
+    }
     const bool phased = phased_rows<Op>::value && !vec && phase0 >= 0 && T % 4 != 0;
     e = dispatch_store_policy<Op, Kernel::kChain>(E, T, [&](auto sp) {
       constexpr int SP = decltype(sp)::value;
@@ -634,9 +695,8 @@ int launch(const Op& op, int64_t E, int64_t T, bool vec, void* workspace, size_t
     });
   } else if (strided_rows<Op>::value && vec && T > kShortMaxT / 2) {
     if constexpr (strided_rows<Op>::value) {
-      e = dispatch_store_policy<Op, Kernel::kStrided>(E, T, [&](auto sp) {
-        return launch_strided<Op, decltype(sp)::value>(op, E, Ti, s);
-      });
+      static_assert(kStridedThreads * kSeg * kStridedSegments == kShortMaxT, "one row per workgroup");
+      e = launch_strided<Op, kStridedThreads, kStridedSegments, kAligned>(op, E, Ti, kStridedThreads, s);
     }
   } else {
     e = dispatch_store_policy<Op, Kernel::kRows>(E, T, [&](auto sp) {
