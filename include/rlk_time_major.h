@@ -1,6 +1,6 @@
 /*
- * rlk_time_major.h -- calls on time-major arrays, between the PyTorch extension and
- * librl_triton_amd.so (not part of the C ABI of rl_triton_amd.h).
+ * rlk_time_major.h -- calls on time-major arrays, and normalised GAE in one launch, between the
+ * PyTorch extension and librl_triton_amd.so (not part of the C ABI of rl_triton_amd.h).
  *
  * A call's [num_envs, seq_len] inputs are transposed views of [seq_len, num_envs] buffers:
  * element (env, t) at env + t * step_stride of every array (Retrace's action rows at
@@ -44,6 +44,8 @@ typedef struct rlk_time_major_call {
   float rho_bar, c_bar, eps;
   void *partials;       /* RLK_OP_GAE_NORMALIZED: rlk_time_major_partials_bytes bytes */
   size_t partials_bytes;
+  void *sync;           /* RLK_OP_GAE_NORMALIZED in one launch, or NULL: see below */
+  uint32_t epoch;
 } rlk_time_major_call;
 
 /* 1 if calls of this shape are taken (rlk_time_major returns RLK_ERR_INVALID_ARGUMENT for
@@ -53,6 +55,18 @@ typedef struct rlk_time_major_call {
 int rlk_time_major_takes(int64_t num_envs, int64_t seq_len, int64_t step_stride, int64_t num_actions);
 size_t rlk_time_major_partials_bytes(int64_t num_envs, int64_t seq_len);
 int rlk_time_major(const rlk_time_major_call *call, void *stream);
+
+/* Normalised GAE in one launch (step_stride ignored: contiguous rows; rlk_time_major takes the
+ * same two fields).  sync: RLK_NORM_SYNC_BYTES of device memory, zero-filled once, for calls
+ * ordered on one stream; epoch: 1 to RLK_NORM_MAX_EPOCH and different from every earlier call's on
+ * it since it was zeroed (so not for graph capture, whose replays would repeat it).  Returns 1,
+ * with nothing launched, for calls whose workgroups do not all fit the GPU at once, rows split
+ * into tiles and time-major rows of more than one pass: those take two launches. */
+#define RLK_NORM_SYNC_BYTES (8 * (8 + 4 * 256 + 256))
+#define RLK_NORM_MAX_EPOCH 0xffff
+int rlk_gae_normalized_one_launch(const rlk_time_major_call *call, void *stream);
+/* 0: no call of this shape takes one launch (a quick look, in either layout). */
+int rlk_gae_normalized_one_launch_takes(int64_t num_envs, int64_t seq_len);
 
 #ifdef __cplusplus
 }

@@ -17,7 +17,7 @@ ColumnShape column_shape(int64_t num_envs, int64_t T, int max_waves) {
   constexpr int wave_steps = 4 * kWave / kCols;
   const int64_t passes = (T + max_waves * wave_steps - 1) / (max_waves * wave_steps);
   const int waves = (int)((T + passes * wave_steps - 1) / (passes * wave_steps));
-  const int groups = waves >= 4 ? 1 : 4 / waves;
+  const int groups = (4 + waves - 1) / waves;
   const int64_t col_groups = (num_envs + kCols - 1) / kCols;
   return {waves, groups, (col_groups + groups - 1) / groups};
 }
@@ -34,10 +34,7 @@ int launch_columns(const Op& op, const rlk_time_major_call& c, hipStream_t strea
   int64_t n = c.num_envs, ld = c.step_stride;
   int T = (int)c.seq_len, waves = sh.waves;
   void* args[] = {const_cast<Op*>(&op), &n, &T, &ld, &waves};
-  return hipLaunchKernel(reinterpret_cast<const void*>(&columns_kernel<Op>),
-                         dim3((unsigned)sh.blocks), dim3(threads), args, dynamic_lds(op, threads), stream) == hipSuccess
-             ? RLK_OK
-             : RLK_ERR_LAUNCH;
+  return status_of(launch_kernel(reinterpret_cast<const void*>(&columns_kernel<Op>), op, sh.blocks, threads, args, stream));
 }
 
 // Rows above 2048 steps are few and are split over workgroups, which the row kernels do.  Retrace
@@ -57,6 +54,11 @@ E* out_of(const rlk_time_major_call& c, int i) { return static_cast<E*>(c.out[i]
 template <class StatsOp>
 int launch_normalized(StatsOp op, const rlk_time_major_call& c, hipStream_t stream) {
   using E = typename StatsOp::Elem;
+  if (c.sync != nullptr) {
+    const ColumnShape sh = column_shape(c.num_envs, c.seq_len, column_waves<StatsOp>::value);
+    if (c.seq_len > 4 * kWave / kCols * sh.waves) return kNotTaken;  // more than one pass
+    return launch_columns(OneLaunchOp<StatsOp>{op, one_launch(c)}, c, stream);
+  }
   const int64_t blocks = column_blocks<StatsOp>(c.num_envs, c.seq_len);
   op.partials = static_cast<double*>(c.partials);
   if (!partials_fit(c.partials, c.partials_bytes, blocks)) return RLK_ERR_WORKSPACE;

@@ -103,8 +103,11 @@ __global__ __launch_bounds__(column_waves<Op>::value* kWave) void columns_kernel
   const int groups = (int)(blockDim.x / kWave) / waves;
   // Workgroups go to the 8 XCDs in turn; an XCD takes consecutive column groups, so that the
   // halves of a 128-byte line are read through one L2.
-  const unsigned nb = gridDim.x, xcd = blockIdx.x & 7u, per = nb >> 3, rest = nb & 7u;
-  const unsigned block = xcd * per + (xcd < rest ? xcd : rest) + (blockIdx.x >> 3);
+  auto block_of = [](unsigned b) {
+    const unsigned xcd = b & 7u, per = gridDim.x >> 3, rest = gridDim.x & 7u;
+    return xcd * per + (xcd < rest ? xcd : rest) + (b >> 3);
+  };
+  const unsigned block = block_of(blockIdx.x);
   const int64_t col0 = ((int64_t)block * groups + group) * COLS;
   const bool active = col0 + (lane & (COLS - 1)) < E;
   const int64_t row = active ? col0 + (lane & (COLS - 1)) : E - 1;  // idle lanes read the last column
@@ -164,6 +167,23 @@ __global__ __launch_bounds__(column_waves<Op>::value* kWave) void columns_kernel
     if (c == 0) x_in = x;
     State xs[S];
     replay<FWD, S>(steps, x_in, xs);
+    if constexpr (in_one_launch<Op>::value) {  // (the launcher: one pass)
+      if (active) {
+        op.template emit_returns<S, kElementAligned, 0>(R, xs, row, t0, T);
+        op.template stats<S>(R, xs, t0, T, st);
+      }
+      finish_normalized<MAXW * kWave>(
+          op.one, st, op.out, (int)(blockDim.x / kWave),
+          [&](auto f) {
+            if (active) op.template emit_advantages<S, kElementAligned, 0>(f, xs, row, t0, T);
+          },
+          [&](int j, int64_t& first, int64_t& count) {
+            const int64_t rows = (int64_t)groups * COLS, r0 = block_of(j) * rows;
+            first = r0 * T;
+            count = r0 >= E ? 0 : (E - r0 < rows ? E - r0 : rows) * T;
+          });
+      return;
+    }
     if (active) {
       op.template emit<S, kElementAligned>(R, h, xs, x_in, row, t0, T);
       if constexpr (Op::kBlockStats) op.template stats<S>(R, xs, t0, T, st);

@@ -542,6 +542,19 @@ __device__ __forceinline__ uint64_t pack(uint32_t tag, float v) {
   return ((uint64_t)tag << 32) | (uint64_t)__float_as_uint(v);
 }
 
+// s_waitcnt vmcnt(0): the wave's own memory operations are complete.  (In the look-back: before
+// its path rejoins the other waves', so nothing it issued looks pending to the compiler.)
+__device__ __forceinline__ void wait_vmem() { __builtin_amdgcn_s_waitcnt(0x0F70); }
+
+// Lane L's value of a 64-bit register, in every lane.
+template <int L>
+__device__ __forceinline__ uint64_t lane_u64(uint64_t x) {
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)x, L);
+  const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(x >> 32), L);
+  return ((uint64_t)hi << 32) | lo;
+}
+__device__ __forceinline__ uint64_t lane0_u64(uint64_t x) { return lane_u64<0>(x); }
+
 // ---------------------------------------------------------------------------------------
 // Segment pieces shared by both kernels.
 // ---------------------------------------------------------------------------------------
@@ -636,6 +649,19 @@ __device__ __forceinline__ double wave_total(double v) {
   return v;
 }
 
+// The waves' values s[0 .. waves), summed in index order.  All reads at once: a loop over a
+// run-time count waits for each (1 us for three statistics of eight waves).
+template <int NW>
+__device__ __forceinline__ double sum_waves(const double (&s)[NW], int waves) {
+  double v[NW];
+#pragma unroll
+  for (int w = 0; w < NW; ++w) v[w] = s[w];
+  double a = 0.0;
+#pragma unroll
+  for (int w = 0; w < NW; ++w) a += w < waves ? v[w] : 0.0;
+  return a;
+}
+
 // Every thread of the workgroup calls this once; thread 0 writes
 // partials[kStatWords*blockIdx.x + {0,1,2}] = {n, sum, sum of squares}.
 // (waves: the workgroup's, where it may have fewer than NT threads).
@@ -653,11 +679,8 @@ __device__ __forceinline__ void block_stats(Stats st, double* __restrict__ parti
     s_st[2][wave] = st.sq;
   }
   __syncthreads();
-  if (threadIdx.x < kStatWords) {
-    double a = 0.0;
-    for (int w = 0; w < waves; ++w) a += s_st[threadIdx.x][w];
-    partials[kStatWords * blockIdx.x + threadIdx.x] = a;
-  }
+  if (threadIdx.x < kStatWords)
+    partials[kStatWords * blockIdx.x + threadIdx.x] = sum_waves<NW>(s_st[threadIdx.x], waves);
 }
 
 // One level of a tree over the partials, for first launches of many workgroups: workgroup j
@@ -689,6 +712,16 @@ __global__ __launch_bounds__(NT) void reduce_partials_kernel(const double* __res
     st.sq += p[k][2];
   }
   block_stats<NT>(st, out);
+}
+
+// Mean and std + eps from the statistics' totals (std unbiased, count - 1, as torch's x.std()).
+__device__ __forceinline__ void mean_and_scale(double n, double sum, double sq, float eps, float& m, float& d) {
+  const double mean = sum / n;  // nan when nothing was counted
+  double var = (sq - sum * mean) / (n - 1.0);
+  var = var > 0.0 ? var : 0.0;
+  if (!(n >= 2.0)) var = __builtin_nan("");  // torch: the unbiased std of one element is nan
+  m = (float)mean;
+  d = (float)sqrt(var) + eps;
 }
 
 // Second launch of the normalisation: every workgroup combines the per-workgroup partials
@@ -748,12 +781,8 @@ __global__ __launch_bounds__(NT) void normalize_kernel(E* __restrict__ x,
     sum += s_st[1][w];
     sq += s_st[2][w];
   }
-  const double mean = sum / n;  // nan when nothing was counted
-  double var = (sq - sum * mean) / (n - 1.0);
-  var = var > 0.0 ? var : 0.0;
-  if (!(n >= 2.0)) var = __builtin_nan("");  // torch: the unbiased std of one element is nan
-  const float m = (float)mean;
-  const float d = (float)sqrt(var) + eps;
+  float m, d;
+  mean_and_scale(n, sum, sq, eps, m, d);
   if constexpr (VEC) {
     for (int64_t i = first; i < units; i += stride) {
       float4 v = i == first ? v0 : load_quad<true>(x + 4 * i);
@@ -766,6 +795,196 @@ __global__ __launch_bounds__(NT) void normalize_kernel(E* __restrict__ x,
   } else {
     for (int64_t i = first; i < units; i += stride)
       store_one_nt(x + i, ((i == first ? v0.x : load_one_nt(x + i)) - m) / d);
+  }
+}
+
+// ---------------------------------------------------------------------------------------
+// The normalisation in the scan's own launch, for calls whose workgroups are all resident at
+// once (the launcher's choice): each workgroup keeps its advantages in registers, publishes its
+// statistics, waits for every other workgroup's and stores the normalised values.  Against two
+// launches this saves writing and reading the raw advantages and one launch's host and device
+// time.
+//
+// Nothing depends on residency.  The wait is bounded: a workgroup that does not see all
+// statistics in `polls` reads stores its raw advantages, marks itself raw, looks once more and
+// leaves.  Every workgroup that did see them all looks at the end, after its own statistics are
+// visible, whether any is marked, and normalises the marked ones it can claim.  None is missed:
+// a workgroup that marks itself and then still misses some statistics did so before these became
+// visible, so their publisher, looking after that, sees the mark; and the one whose statistics
+// become visible last sees everybody's.
+//
+// Every workgroup reads every other's statistics itself, one thread each (at most 256
+// workgroups), and sums them in normalize_kernel's order: the same bits.  A sum by whoever comes
+// last, published for the others, is two more trips through memory, and everybody then reads the
+// same few lines.
+//
+// sync (uint64 words, zeroed once): [0] "some workgroup is raw"; from kNormFirst on kNormWords words
+// per workgroup, {16 bits of the epoch | 48 bits of its statistics}; from kNormStates on a state
+// word per workgroup.  The epoch is counted by the host per buffer from 1 and the buffer zeroed
+// again before it wraps: nothing is reset between calls.  (Word k of all workgroups side by side,
+// eight workgroups to a line, took 2 us longer at 256 of them; 64 bytes apart 0.1 us longer.)
+//
+// Bound by the trips of the statistics through memory between the XCDs.  Calls in a row, us per
+// call, two launches -> one: [64,64] 9.4 -> 4.7, [1024,128] 9.2 -> 4.9, [4096,128] 9.2 -> 7.5 (all
+// paced by the host before; on the device 7.1 -> 7.3), [256,4096] 11.4 -> 9.0, [256,8192]
+// 17.3 -> 11.6, [200,12000] 18.5 -> 12.1.
+constexpr int kNormWords = 4;  // three doubles in 4 x 48 bits
+constexpr int kNormMaxBlocks = 256;  // a thread polls for each
+constexpr int kNormFirst = 8, kNormStates = kNormFirst + kNormWords * kNormMaxBlocks;
+constexpr int kNormSyncWords = kNormStates + kNormMaxBlocks;
+constexpr uint32_t kNormMaxEpoch = 0xffff;
+constexpr uint64_t kNormRaw = 1, kNormClaimed = 2;
+
+struct OneLaunch {
+  uint64_t* sync;
+  uint32_t epoch;
+  int polls;
+  float eps;
+};
+
+// A statistics op that finishes in its own launch.
+template <class StatsOp>
+struct OneLaunchOp : StatsOp {
+  OneLaunch one;
+};
+template <class Op>
+struct in_one_launch : std::false_type {};
+template <class StatsOp>
+struct in_one_launch<OneLaunchOp<StatsOp>> : std::true_type {};
+
+// st: the thread's statistics.  store(f): stores f(advantage) for every advantage the thread
+// holds (E rounds to the storage type as the raw store of two launches would).  region(j, first,
+// count): where workgroup j's advantages lie in x.  Called by every thread, at least
+// kNormMaxBlocks of them.
+template <int NT, class E, class Store, class Region>
+__device__ __forceinline__ void finish_normalized(const OneLaunch& one, Stats st, E* __restrict__ x, int waves,
+                                                  Store store, Region region) {
+  constexpr int NW = NT / kWave, PW = kNormMaxBlocks / kWave;
+  constexpr uint64_t kLow48 = (uint64_t{1} << 48) - 1;
+  static_assert(NW >= PW, "a thread per workgroup");
+  __shared__ double s_own[kStatWords][NW], s_all[kStatWords][PW];
+  __shared__ int s_seen[PW];
+  __shared__ int s_claimed[kNormMaxBlocks];
+  __shared__ int s_nclaimed;
+  const int tid = threadIdx.x, lane = __lane_id(), wave = tid / kWave;
+  const int nb = (int)gridDim.x, own = (int)blockIdx.x;
+  auto line = [&](int j) { return one.sync + kNormFirst + kNormWords * j; };
+  uint64_t* const state = one.sync + kNormStates;
+  const uint64_t tag = (uint64_t)one.epoch << 48;
+
+  st.n = wave_total(st.n);
+  st.sum = wave_total(st.sum);
+  st.sq = wave_total(st.sq);
+  if (lane == kWave - 1) {
+    s_own[0][wave] = st.n;
+    s_own[1][wave] = st.sum;
+    s_own[2][wave] = st.sq;
+  }
+  __syncthreads();
+  if (wave == 0) {
+    // statistic k in lane k; words 0..2: the low 48 bits of a statistic each, word 3: their high
+    // 16 bits
+    const uint64_t u = (uint64_t)__double_as_longlong(sum_waves<NW>(s_own[lane < kStatWords ? lane : 0], waves));
+    const uint64_t high = lane_u64<0>(u) >> 48 | lane_u64<1>(u) >> 48 << 16 | lane_u64<2>(u) >> 48 << 32;
+    if (lane < kNormWords) atomic_st(line(own) + lane, tag | (lane < kStatWords ? u & kLow48 : high));
+  }
+  // All statistics into s_all; false if some are missing after `polls` more reads.
+  auto gather = [&](int polls) -> bool {
+    if (wave < PW) {
+      uint64_t v[kNormWords];
+      bool here = tid >= nb;
+      for (int p = 0;; ++p) {
+        if (!here) {
+#pragma unroll
+          for (int i = 0; i < kNormWords; ++i) v[i] = atomic_ld(line(tid) + i);
+          here = true;
+#pragma unroll
+          for (int i = 0; i < kNormWords; ++i) here = here && (v[i] & ~kLow48) == tag;
+        }
+        if (__ballot(!here) == 0 || p >= polls) break;
+        __builtin_amdgcn_s_sleep(1);
+      }
+      const bool seen = __ballot(!here) == 0;
+      wait_vmem();  // wave 0: this workgroup's statistics are visible
+      asm volatile("" : : : "memory");
+      if (lane == 0) s_seen[wave] = seen;
+#pragma unroll
+      for (int k = 0; k < kStatWords; ++k) {
+        double a = 0.0;
+        if (seen && tid < nb)
+          a += __longlong_as_double((long long)((v[k] & kLow48) | (v[kNormWords - 1] >> (16 * k)) << 48));
+        a = wave_total(a);
+        if (lane == kWave - 1) s_all[k][wave] = a;
+      }
+    }
+    __syncthreads();
+    bool seen = true;
+#pragma unroll
+    for (int w = 0; w < PW; ++w) seen = seen && s_seen[w] != 0;
+    return seen;
+  };
+  auto totals = [&](float& m, float& d) {
+    double t[kStatWords] = {0.0, 0.0, 0.0};
+#pragma unroll
+    for (int w = 0; w < PW; ++w) {
+#pragma unroll
+      for (int k = 0; k < kStatWords; ++k) t[k] += s_all[k][w];
+    }
+    mean_and_scale(t[0], t[1], t[2], one.eps, m, d);
+  };
+  float m = 0.f, d = 1.f;
+  auto normalized = [&](float a) { return (to_f32(from_f32<E>(a)) - m) / d; };
+  uint64_t look = 0;  // the "some workgroup is raw" word, read once what this workgroup published is visible
+  if (!gather(one.polls)) {
+    store([](float a) { return a; });
+    __threadfence();
+    __syncthreads();
+    if (tid == 0) {
+      atomic_st(state + own, tag | kNormRaw);
+      atomic_st(one.sync, tag | kNormRaw);
+      __threadfence();
+    }
+    __syncthreads();
+    if (!gather(0)) return;
+    if (tid == 0) {
+      uint64_t raw = tag | kNormRaw;
+      s_nclaimed = __hip_atomic_compare_exchange_strong(state + own, &raw, tag | kNormClaimed, __ATOMIC_ACQ_REL,
+                                                        __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      look = atomic_ld(one.sync);
+    }
+    __syncthreads();
+    const int mine = s_nclaimed;
+    __syncthreads();
+    totals(m, d);
+    if (mine) store(normalized);
+  } else {
+    if (tid == 0) look = atomic_ld(one.sync);
+    totals(m, d);
+    store(normalized);
+  }
+  if (tid == 0) s_nclaimed = look == (tag | kNormRaw);
+  __syncthreads();
+  if (s_nclaimed == 0) return;
+  __syncthreads();
+  if (tid == 0) s_nclaimed = 0;
+  __syncthreads();
+  if (tid < nb) {
+    uint64_t raw = tag | kNormRaw;
+    if (atomic_ld(state + tid) == raw &&
+        __hip_atomic_compare_exchange_strong(state + tid, &raw, tag | kNormClaimed, __ATOMIC_ACQ_REL,
+                                             __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+      s_claimed[atomicAdd(&s_nclaimed, 1)] = tid;
+  }
+  __syncthreads();
+  const int claimed = s_nclaimed;
+  __threadfence();  // the claimed workgroups' raw values, stored before their marks
+  for (int c = 0; c < claimed; ++c) {
+    int64_t first, count;
+    region(s_claimed[c], first, count);
+    for (int64_t i = tid; i < count; i += blockDim.x) {
+      const float v = to_f32(x[first + i]);
+      x[first + i] = from_f32<E>((v - m) / d);
+    }
   }
 }
 
@@ -894,8 +1113,26 @@ __global__ __launch_bounds__(NT) void rows_kernel(const Op op, int64_t E, int T,
   if ((li & (W - 1)) == 0) x_in = carry;
   State xs[S];
   replay<FWD, S>(steps, x_in, xs);
+  if constexpr (in_one_launch<Op>::value) {
+    Stats st;
+    if (active) {
+      op.template stats<S>(R, xs, t0, T, st);
+      op.template emit_returns<S, VEC, SP>(R, xs, row, t0, T);
+    }
+    finish_normalized<NT>(
+        op.one, st, op.out, NW,
+        [&](auto f) {
+          if (active) op.template emit_advantages<S, VEC, SP>(f, xs, row, t0, T);
+        },
+        [&](int j, int64_t& first, int64_t& count) {
+          const int64_t rows = NT >> log2L, r0 = j * rows;
+          first = r0 * T;
+          count = (E - r0 < rows ? E - r0 : rows) * T;
+        });
+    return;
+  }
   if (active) op.template emit<S, VEC, SP>(R, h, xs, x_in, row, t0, T);
-  if constexpr (Op::kBlockStats) {
+  if constexpr (Op::kBlockStats && !in_one_launch<Op>::value) {
     Stats st;
     if (active) op.template stats<S>(R, xs, t0, T, st);
     block_stats<NT>(st, op.partials);
@@ -978,17 +1215,6 @@ __global__ __launch_bounds__(NT) void rows_pair_kernel(const Op op, int64_t E, i
 // Long rows: the decoupled look-back.
 // ---------------------------------------------------------------------------------------
 __host__ __device__ inline int lookback_slots(int64_t E) { return E < kSlots ? (int)E : kSlots; }
-
-// s_waitcnt vmcnt(0): the look-back wave's own traffic is complete before its path rejoins
-// the other waves', so nothing it issued looks pending to the compiler afterwards.
-__device__ __forceinline__ void wait_vmem() { __builtin_amdgcn_s_waitcnt(0x0F70); }
-
-// Lane 0's value of a 64-bit register, in every lane.
-__device__ __forceinline__ uint64_t lane0_u64(uint64_t x) {
-  const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)x, 0);
-  const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(x >> 32), 0);
-  return ((uint64_t)hi << 32) | lo;
-}
 
 // What one look-back read finds for a tile: lane l examines tile k -/+ (1 + base + l) of
 // the row, in its own status words (st) and in those another workgroup published for it
@@ -1350,6 +1576,26 @@ __global__ __launch_bounds__(NT) void rows_strided_kernel(const Op op, int64_t E
     carry = lane_bcast(lane_scan(pm, NW), NW - 1).apply(carry);
   }
   Stats st;
+  if constexpr (in_one_launch<Op>::value) {
+    State xs[Q][S];
+#pragma unroll
+    for (int r = 0; r < Q; ++r) {
+      State x_in = lane_prev(m[r].apply(carry));
+      if (lane == 0) x_in = carry;
+      carry = rowagg[r].apply(carry);
+      replay<FWD, S>(steps[r], x_in, xs[r]);
+      op.template emit_returns<S, VEC, SP>(R[r], xs[r], row, seg_t0(r), T);
+      op.template stats<S>(R[r], xs[r], seg_t0(r), T, st);
+    }
+    finish_normalized<NT>(
+        op.one, st, op.out, nw,
+        [&](auto f) {
+#pragma unroll
+          for (int r = 0; r < Q; ++r) op.template emit_advantages<S, VEC, SP>(f, xs[r], row, seg_t0(r), T);
+        },
+        [&](int j, int64_t& first, int64_t& count) { first = (int64_t)j * T, count = T; });
+    return;
+  }
 #pragma unroll
   for (int r = 0; r < Q; ++r) {
     State x_in = lane_prev(m[r].apply(carry));

@@ -70,12 +70,53 @@ int gae_normalized_impl(const E* rewards, const E* values, const E* terminateds,
                                    returns, nullptr});
 }
 
+static_assert(RLK_NORM_SYNC_BYTES == kNormSyncWords * sizeof(uint64_t) && RLK_NORM_MAX_EPOCH == kNormMaxEpoch,
+              "the sync buffer's layout");
+
+// One launch, or kNotTaken.
+template <class E>
+int one_launch_impl(const rlk_time_major_call& c, void* stream) {
+  auto in = [&](int i) { return static_cast<const E*>(c.in[i]); };
+  E *adv = static_cast<E*>(c.out[0]), *ret = static_cast<E*>(c.out[1]);
+  if (!in(0) || !in(1) || !in(2) || !adv || !ret || !c.sync || c.epoch == 0 || c.epoch > kNormMaxEpoch ||
+      !valid_boot(c.bootstrap, c.boot_mode))
+    return RLK_ERR_INVALID_ARGUMENT;
+  const E* boot = c.boot_mode == RLK_BOOT_NONE ? nullptr : static_cast<const E*>(c.bootstrap);
+  const bool vec = c.seq_len % 4 == 0 && quad_aligned(in(0), in(1), in(2), in(3), in(4), adv, ret) &&
+                   (c.boot_mode != RLK_BOOT_FULL || quad_aligned(boot));
+  const float gl = c.gamma * c.lambda_;
+  auto run = [&](auto op) {
+    return launch(OneLaunchOp<decltype(op)>{op, one_launch(c)}, c.num_envs, c.seq_len, vec, nullptr, 0, stream);
+  };
+  if (in(4)) {
+    if (in(3))
+      return run(MaskedGaeStatsOp<true, E>{{in(0), in(1), in(2), in(3), boot, in(4), adv, c.boot_mode, c.gamma, gl},
+                                           ret, nullptr});
+    return run(MaskedGaeStatsOp<false, E>{{in(0), in(1), in(2), nullptr, boot, in(4), adv, c.boot_mode, c.gamma, gl},
+                                          ret, nullptr});
+  }
+  if (in(3))
+    return run(GaeStatsOp<true, E>{{in(0), in(1), in(2), in(3), boot, adv, c.boot_mode, c.gamma, gl}, ret, nullptr});
+  return run(GaeStatsOp<false, E>{{in(0), in(1), in(2), nullptr, boot, adv, c.boot_mode, c.gamma, gl}, ret, nullptr});
+}
+
 }  // namespace
 }  // namespace rlk
 
 using namespace rlk;
 
 extern "C" {
+
+int rlk_gae_normalized_one_launch_takes(int64_t num_envs, int64_t seq_len) {
+  // A workgroup holds at most 4096 advantages of short rows, or one whole longer row.
+  if (seq_len <= kShortMaxT) return num_envs * seq_len <= (int64_t)kNormMaxBlocks * 4096;
+  return num_envs <= kNormMaxBlocks && whole_row_segments<GaeStatsOp<true>>(num_envs, seq_len, true) > 0;
+}
+
+int rlk_gae_normalized_one_launch(const rlk_time_major_call* call, void* stream) {
+  if (is_empty(call->num_envs, call->seq_len)) return kNotTaken;
+  return call->bf16 ? one_launch_impl<bf16>(*call, stream) : one_launch_impl<float>(*call, stream);
+}
 
 size_t rlk_gae_normalized_partials_bytes(int64_t num_envs, int64_t seq_len) {
   return gae_normalized_partials(num_envs, seq_len);

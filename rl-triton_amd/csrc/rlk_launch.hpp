@@ -5,6 +5,9 @@
 #include <hip/hip_runtime.h>
 
 #include <atomic>
+#include <map>
+#include <mutex>
+#include <utility>
 
 #include "rl_triton_amd.h"
 #include "rlk_ops.hpp"
@@ -327,6 +330,34 @@ struct paired_rows : std::false_type {};
 template <int NA, bool TRUNC>
 struct paired_rows<RetraceOp<NA, TRUNC, float>> : std::bool_constant<(NA > 0)> {};
 
+// Whether a launch's workgroups all fit the GPU at once (for the normalisation in the scan's own
+// launch; a wrong answer costs time, not results).  The runtime's answer per kernel and
+// workgroup size is kept.
+inline bool all_resident(const void* kernel, int64_t blocks, int threads, size_t lds) {
+  static std::mutex mu;
+  static std::map<std::pair<const void*, int>, int> per_cu;
+  if (blocks > kNormMaxBlocks || threads < kNormMaxBlocks) return false;
+  std::lock_guard<std::mutex> lock(mu);
+  auto it = per_cu.find({kernel, threads});
+  if (it == per_cu.end()) {
+    int n = 0;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, kernel, threads, lds) != hipSuccess) n = 0;
+    it = per_cu.emplace(std::make_pair(kernel, threads), n).first;
+  }
+  return blocks <= (int64_t)it->second * device_cus();
+}
+
+// A kernel launch of an op.  hipErrorNotReady, and nothing launched: a OneLaunchOp's workgroups do
+// not fit at once.
+template <class Op>
+hipError_t launch_kernel(const void* kernel, const Op& op, int64_t blocks, int threads, void** args, hipStream_t stream) {
+  const size_t lds = dynamic_lds(op, threads);
+  if constexpr (in_one_launch<Op>::value) {
+    if (!all_resident(kernel, blocks, threads, lds)) return hipErrorNotReady;
+  }
+  return hipLaunchKernel(kernel, dim3((unsigned)blocks), dim3(threads), args, lds, stream);
+}
+
 template <class Op, int NT, int S, int VEC, int SP>
 hipError_t launch_rows(const Op& op, int64_t E, int T, hipStream_t stream) {
   int log2L = ceil_log2((T + S - 1) / S);
@@ -346,7 +377,7 @@ hipError_t launch_rows(const Op& op, int64_t E, int T, hipStream_t stream) {
     else if (log2L == 5) k = reinterpret_cast<const void*>(&rows_kernel<Op, NT, S, VEC, 32, SP>);
     else if (log2L >= 6) k = reinterpret_cast<const void*>(&rows_kernel<Op, NT, S, VEC, kWave, SP>);
   }
-  return hipLaunchKernel(k, dim3((unsigned)grid), dim3(NT), args, dynamic_lds(op, NT), stream);
+  return launch_kernel(k, op, grid, NT, args, stream);
 }
 
 // Aligned rows of 1025..2048 steps: one row per 256-thread workgroup, two wave-strided
@@ -371,8 +402,8 @@ hipError_t launch_strided(const Op& op, int64_t E, int T, int threads, hipStream
   if (E * threads > 0xffffffffLL) return hipErrorInvalidValue;  // launch() splits such calls
   int unused = 0;
   void* args[] = {const_cast<Op*>(&op), &E, &T, &unused};
-  return hipLaunchKernel(reinterpret_cast<const void*>(&rows_strided_kernel<Op, NT, Q, VEC, 1>),
-                         dim3((unsigned)E), dim3(threads), args, 0, stream);
+  return launch_kernel(reinterpret_cast<const void*>(&rows_strided_kernel<Op, NT, Q, VEC, 1>), op, E, threads, args,
+                       stream);
 }
 
 template <class Op, int VEC>
@@ -481,6 +512,8 @@ template <bool TRUNC, class E>
 struct n_outputs<GaeStatsOp<TRUNC, E>> : std::integral_constant<int, 2> {};
 template <bool TRUNC, class E>
 struct n_outputs<MaskedGaeStatsOp<TRUNC, E>> : std::integral_constant<int, 2> {};
+template <class StatsOp>
+struct n_outputs<OneLaunchOp<StatsOp>> : n_outputs<StatsOp> {};
 template <class Op>
 struct long_rows_write_through : std::true_type {};
 template <bool TRUNC, class E>
@@ -645,6 +678,12 @@ int64_t call_blocks(int64_t E, int64_t T) {
   return total;
 }
 
+// launch()'s answer to a OneLaunchOp where the call is not one for it.
+constexpr int kNotTaken = 1;
+inline int status_of(hipError_t e) {
+  return e == hipSuccess ? RLK_OK : e == hipErrorNotReady ? kNotTaken : RLK_ERR_LAUNCH;
+}
+
 // vec: kAligned access.  phase0 >= 0: the element phase every [E, T] array of the call
 // shares at row 0 (common_phase), for the phased access of long rows when T % 4 != 0.
 template <class Op>
@@ -653,7 +692,9 @@ int launch(const Op& op, int64_t E, int64_t T, bool vec, void* workspace, size_t
   if (E < 0 || T < 0 || T > (int64_t{1} << 30)) return RLK_ERR_INVALID_ARGUMENT;
   if (E == 0 || T == 0) return RLK_OK;
   const int64_t rows = rows_per_launch<Op>(E, T, vec);
-  if (rows < E) {
+  if constexpr (in_one_launch<Op>::value) {
+    if (rows < E) return kNotTaken;
+  } else if (rows < E) {
     int64_t blocks = 0;  // the statistics ops' partials of the ranges before this one
     for (int64_t r0 = 0; r0 < E; r0 += rows) {
       const int64_t n = rows < E - r0 ? rows : E - r0;
@@ -672,18 +713,19 @@ int launch(const Op& op, int64_t E, int64_t T, bool vec, void* workspace, size_t
   hipError_t e = hipErrorInvalidValue;
   if (T > kShortMaxT) {
     uint64_t* ws = reinterpret_cast<uint64_t*>(workspace);
-    if (ws == nullptr || workspace_bytes_given < workspace_bytes(E, T) || !aligned16(ws))
+    if (!in_one_launch<Op>::value && (ws == nullptr || workspace_bytes_given < workspace_bytes(E, T) || !aligned16(ws)))
       return RLK_ERR_WORKSPACE;
     if constexpr (whole_row<Op>::value != WholeRow::kNever) {
       const int segments = whole_row_segments<Op>(E, T, vec);
       if (segments > 0) {
         e = vec ? launch_whole_row<Op, kAligned>(op, E, Ti, segments, s)
                 : launch_whole_row<Op, kElementAligned>(op, E, Ti, segments, s);
-        return e == hipSuccess ? RLK_OK : RLK_ERR_LAUNCH;
+        return status_of(e);
       }
     }
+    if constexpr (in_one_launch<Op>::value) return kNotTaken;
     const bool phased = phased_rows<Op>::value && !vec && phase0 >= 0 && T % 4 != 0;
-    e = dispatch_store_policy<Op, Kernel::kChain>(E, T, [&](auto sp) {
+    if constexpr (!in_one_launch<Op>::value) e = dispatch_store_policy<Op, Kernel::kChain>(E, T, [&](auto sp) {
       constexpr int SP = decltype(sp)::value;
       if constexpr (phased_rows<Op>::value) {
         if (phased) return launch_long<Op, kPhased, SP>(op, E, Ti, ws, s, phase0);
@@ -717,7 +759,7 @@ int launch(const Op& op, int64_t E, int64_t T, bool vec, void* workspace, size_t
                     : launch_rows<Op, kNTWide, 4, kElementAligned, SP>(op, E, Ti, s);
     });
   }
-  return e == hipSuccess ? RLK_OK : RLK_ERR_LAUNCH;
+  return status_of(e);
 }
 
 // Empty shapes are a successful no-op (their data pointers may be null); negative sizes

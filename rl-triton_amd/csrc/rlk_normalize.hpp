@@ -2,6 +2,7 @@
 // statistics to the normalised advantages.
 #pragma once
 #include "rlk_launch.hpp"
+#include "rlk_time_major.h"
 
 namespace rlk {
 
@@ -28,6 +29,11 @@ inline int64_t partials_triples(int64_t nparts) {
 inline bool partials_fit(const void* partials, size_t bytes, int64_t nparts) {
   return partials != nullptr && (reinterpret_cast<uintptr_t>(partials) & 7u) == 0 && nparts <= 0x7fffffffLL &&
          bytes >= (size_t)partials_triples(nparts) * kStatWords * sizeof(double);
+}
+
+// The one-launch form a call asks for (c.sync != nullptr).
+inline OneLaunch one_launch(const rlk_time_major_call& c) {
+  return {static_cast<uint64_t*>(c.sync), c.epoch, g_fallback_polls.load(std::memory_order_relaxed), c.eps};
 }
 
 // Rewrites the n advantages as (A - mean) / (std + eps), from the first launch's nparts triples

@@ -117,6 +117,22 @@ struct GaeStatsOp : GaeOp<TRUNC, E> {
   template <int S>
   using Regs = typename GaeOp<TRUNC, E>::template Regs<S>;
 
+  // the two outputs by themselves, advantages mapped by f (OneLaunchOp)
+  template <int S, int VEC, int SP>
+  __device__ void emit_returns(const Regs<S>& R, const float (&xs)[S], int64_t row, int t0, int T) const {
+    float rt[S];
+#pragma unroll
+    for (int i = 0; i < S; ++i) rt[i] = xs[i] + R.v[i];
+    store_seg<S, VEC>(returns + row * (int64_t)T, t0, T, rt, SP != 0);
+  }
+  template <int S, int VEC, int SP, class F>
+  __device__ void emit_advantages(F f, const float (&xs)[S], int64_t row, int t0, int T) const {
+    float a[S];
+#pragma unroll
+    for (int i = 0; i < S; ++i) a[i] = f(xs[i]);
+    store_seg<S, VEC>(this->out + row * (int64_t)T, t0, T, a, SP != 0);
+  }
+
   template <int S, int VEC, int SP = 0>
   __device__ void emit(const Regs<S>& R, float, const float (&xs)[S], float, int64_t row, int t0,
                        int T) const {
@@ -238,6 +254,21 @@ struct MaskedGaeStatsOp : MaskedGaeOp<TRUNC, E> {
   double* partials;
   template <int S>
   using Regs = typename MaskedGaeOp<TRUNC, E>::template Regs<S>;
+
+  template <int S, int VEC, int SP>
+  __device__ void emit_returns(const Regs<S>& R, const NvX (&xs)[S], int64_t row, int t0, int T) const {
+    float rt[S];
+#pragma unroll
+    for (int i = 0; i < S; ++i) rt[i] = xs[i].x + R.v[i];
+    store_seg<S, VEC>(returns + row * (int64_t)T, t0, T, rt, SP != 0);
+  }
+  template <int S, int VEC, int SP, class F>
+  __device__ void emit_advantages(F f, const NvX (&xs)[S], int64_t row, int t0, int T) const {
+    float a[S];
+#pragma unroll
+    for (int i = 0; i < S; ++i) a[i] = f(xs[i].x);
+    store_seg<S, VEC>(this->out + row * (int64_t)T, t0, T, a, SP != 0);
+  }
 
   template <int S, int VEC, int SP = 0>
   __device__ void emit(const Regs<S>& R, NoHalo, const NvX (&xs)[S], NvX, int64_t row, int t0,

@@ -201,6 +201,36 @@ Workspace workspace(const Call& c, const at::Tensor& like) {
   return w;
 }
 
+// The buffers of normalised GAE in one launch, one per (device, stream) like the workspaces, with
+// the count of the calls made on each (its epoch, from 1).  Zero-filled when allocated and again
+// before the count wraps.
+struct NormSync {
+  at::Tensor buf;
+  uint32_t epoch = 0;
+};
+std::map<std::pair<int, uintptr_t>, NormSync>& norm_syncs() {
+  static auto* m = new std::map<std::pair<int, uintptr_t>, NormSync>();
+  return *m;
+}
+
+// Asks for one launch: false for shapes that never take it and while the stream is capturing a
+// graph, whose replays would repeat the epoch.
+bool ask_one_launch(const Call& c, const at::Tensor& like, rlk_time_major_call& t) {
+  if (!rlk_gae_normalized_one_launch_takes(c.E, c.T)) return false;
+  hipStream_t s = static_cast<hipStream_t>(c.stream());
+  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(s, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone) return false;
+  NormSync& n = norm_syncs()[{(int)c.dev, reinterpret_cast<uintptr_t>(s)}];
+  if (!n.buf.defined()) n.buf = at::zeros({(int64_t)RLK_NORM_SYNC_BYTES}, like.options().dtype(at::kByte));
+  if (n.epoch >= std::min<uint64_t>(g_ws_max_calls, RLK_NORM_MAX_EPOCH)) {
+    n.buf.zero_();
+    n.epoch = 0;
+  }
+  t.sync = n.buf.data_ptr();
+  t.epoch = ++n.epoch;
+  return true;
+}
+
 // Typed data pointers (T = float or rlk_bf16) of an input (nullable) and of an output.
 template <class T>
 const T* in_ptr(const at::Tensor* t) {
@@ -347,14 +377,30 @@ PyObject* op_gae_normalized(PyObject* const* a, Py_ssize_t n) {
     rlk_time_major_call t = time_major(c, RLK_OP_GAE_NORMALIZED, in, 5, boot, mode);
     t.gamma = gamma, t.lambda_ = lam, t.eps = eps;
     at::Tensor adv = c.output(*r), ret = c.output(*r);
+    if (ask_one_launch(c, *r, t)) {
+      t.out[0] = adv.data_ptr(), t.out[1] = ret.data_ptr();
+      const int st = rlk_time_major(&t, c.stream());
+      if (st <= 0) return finish(st, "rlk_time_major", pair(adv, ret));
+      t.sync = nullptr;
+    }
     t.partials_bytes = rlk_time_major_partials_bytes(c.E, c.T);
     at::Tensor parts = at::empty({(int64_t)t.partials_bytes}, r->options().dtype(at::kByte));
     t.out[0] = adv.data_ptr(), t.out[1] = ret.data_ptr(), t.partials = parts.data_ptr();
     return finish(rlk_time_major(&t, c.stream()), "rlk_time_major", pair(adv, ret));
   }
+  at::Tensor adv = c.output(*r), ret = c.output(*r);
+  {
+    const at::Tensor* in[] = {r, v, te, tr, mask};
+    rlk_time_major_call t = time_major(c, RLK_OP_GAE_NORMALIZED, in, 5, boot, mode);
+    t.gamma = gamma, t.lambda_ = lam, t.eps = eps;
+    t.out[0] = adv.data_ptr(), t.out[1] = ret.data_ptr();
+    if (ask_one_launch(c, *r, t)) {
+      const int st = rlk_gae_normalized_one_launch(&t, c.stream());
+      if (st <= 0) return finish(st, "rlk_gae_normalized_one_launch", pair(adv, ret));
+    }
+  }
   const Workspace ws = workspace(c, *r);
   if (!ws.ok) return decline();
-  at::Tensor adv = c.output(*r), ret = c.output(*r);
   const size_t pb = rlk_gae_normalized_partials_bytes(c.E, c.T);
   at::Tensor parts = at::empty({(int64_t)(pb > 0 ? pb : 8)}, r->options().dtype(at::kByte));
   const int st = dispatch(c, [&](auto z) {

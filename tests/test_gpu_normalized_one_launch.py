@@ -1,0 +1,98 @@
+"""compute_gae_normalized in one launch (finish_normalized in csrc/rlk_engine.hpp): the bits of the
+two-launch form, also when workgroups stop waiting and leave raw advantages for others to
+normalise."""
+import pytest
+import torch
+
+from _common import make_inputs, to_device
+
+pytestmark = pytest.mark.gpu
+
+# one workgroup, several with a partial last one, one row per workgroup (strided, whole rows), as
+# many workgroups as fit at once and more (two launches), rows split into tiles (two launches)
+SHAPES = [(2, 3), (5, 1), (4, 128), (300, 33), (33, 257), (600, 500), (16, 2048), (300, 1100), (3, 5000),
+          (512, 6000), (200, 9000), (4096, 128), (16384, 128), (20000, 128), (3, 40000)]
+
+
+def _call(d, params, columns=False):
+    import rl_triton
+    if columns:
+        d = {k: v if v is None or v.dim() < 2 else v.t().contiguous().t() for k, v in d.items()}
+    return rl_triton.compute_gae_normalized(d["rewards"], d["values"], d["terminateds"], d.get("truncateds"),
+                                            bootstrap_values=d.get("bootstrap_values"),
+                                            last_value=d.get("last_value"), mask=d.get("mask"), **params)
+
+
+def _two_launches(d, params, columns=False):
+    """The same call captured: graph replays would repeat the one-launch form's call count."""
+    _call(d, params, columns)
+    torch.cuda.synchronize()
+    if columns:
+        d = {k: v if v is None or v.dim() < 2 else v.t().contiguous().t() for k, v in d.items()}
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        out = _call(d, params)
+    g.replay()
+    torch.cuda.synchronize()
+    return [t.clone() for t in out]
+
+
+@pytest.fixture(params=[None, 0, 1], ids=["waiting", "not_waiting", "one_more_read"])
+def polls(request, monkeypatch):
+    """How often a workgroup looks again for the others' statistics: as shipped, never, once."""
+    from rl_triton import _native
+    monkeypatch.delenv("RL_TRITON_CORRECTNESS_WARNINGS", raising=False)
+    lib = _native.load()
+    if request.param is not None:
+        lib.rlk_debug_lookback(-1, request.param)
+    yield request.param
+    lib.rlk_debug_lookback(-1, -1)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["f32", "bf16"])
+@pytest.mark.parametrize("masked", [False, True])
+@pytest.mark.parametrize("shape", SHAPES, ids=lambda s: f"{s[0]}x{s[1]}")
+def test_bits_of_two_launches(shape, masked, dtype, polls, device):
+    op = "gae_normalized_masked" if masked else "gae_normalized"
+    inp, params = make_inputs(op, *shape, seed=sum(shape), p_trunc=0.02, boot="full")
+    d = to_device(inp, device, dtype)
+    want = _two_launches(d, params)
+    for _ in range(5):
+        for g, w in zip(_call(d, params), want):
+            assert torch.equal(g.view(torch.int16), w.view(torch.int16)), f"{op}{shape} {dtype}"
+
+
+@pytest.mark.parametrize("shape", [(5, 3), (100, 33), (300, 100), (4100, 128), (70, 256), (64, 300)],
+                         ids=lambda s: f"{s[0]}x{s[1]}")
+def test_bits_of_two_launches_time_major(shape, polls, device):
+    inp, params = make_inputs("gae_normalized", *shape, seed=7, boot="row")
+    d = to_device(inp, device)
+    want = _two_launches(d, params, columns=True)
+    for _ in range(5):
+        for g, w in zip(_call(d, params, columns=True), want):
+            assert torch.equal(g, w), f"{shape}"
+
+
+def test_streams_and_call_limit(device, monkeypatch):
+    """Calls on two streams at once keep their own buffers; a buffer is zeroed again at the call
+    limit."""
+    from rl_triton import _native
+    monkeypatch.delenv("RL_TRITON_CORRECTNESS_WARNINGS", raising=False)
+    inp, params = make_inputs("gae_normalized", 1024, 128, seed=3, boot="row")
+    d = to_device(inp, device)
+    want = _two_launches(d, params)
+    prev = _native.fast.set_workspace_max_calls(3)
+    try:
+        streams = [torch.cuda.Stream() for _ in range(2)]
+        torch.cuda.synchronize()
+        outs = []
+        for i in range(10):
+            for s in streams:
+                with torch.cuda.stream(s):
+                    outs.append(_call(d, params))
+        torch.cuda.synchronize()
+        for out in outs:
+            for g, w in zip(out, want):
+                assert torch.equal(g, w)
+    finally:
+        _native.fast.set_workspace_max_calls(prev)
