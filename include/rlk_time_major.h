@@ -62,7 +62,7 @@ int rlk_time_major(const rlk_time_major_call *call, void *stream);
  * it since it was zeroed (so not for graph capture, whose replays would repeat it).  Returns 1,
  * with nothing launched, for calls whose workgroups do not all fit the GPU at once, rows split
  * into tiles and time-major rows of more than one pass: those take two launches. */
-#define RLK_NORM_SYNC_BYTES (8 * (8 + 4 * 256 + 256))
+#define RLK_NORM_SYNC_BYTES (8 * (8 + 4 * 512 + 512))
 #define RLK_NORM_MAX_EPOCH 0xffff
 int rlk_gae_normalized_one_launch(const rlk_time_major_call *call, void *stream);
 /* 0: no call of this shape takes one launch (a quick look, in either layout). */

@@ -813,7 +813,7 @@ __global__ __launch_bounds__(NT) void normalize_kernel(E* __restrict__ x,
 // visible, so their publisher, looking after that, sees the mark; and the one whose statistics
 // become visible last sees everybody's.
 //
-// Every workgroup reads every other's statistics itself, one thread each (at most 256
+// Every workgroup reads every other's statistics itself, a thread for one or two (at most 512
 // workgroups), and sums them in normalize_kernel's order: the same bits.  A sum by whoever comes
 // last, published for the others, is two more trips through memory, and everybody then reads the
 // same few lines.
@@ -829,7 +829,8 @@ __global__ __launch_bounds__(NT) void normalize_kernel(E* __restrict__ x,
 // paced by the host before; on the device 7.1 -> 7.3), [256,4096] 11.4 -> 9.0, [256,8192]
 // 17.3 -> 11.6, [200,12000] 18.5 -> 12.1.
 constexpr int kNormWords = 4;  // three doubles in 4 x 48 bits
-constexpr int kNormMaxBlocks = 256;  // a thread polls for each
+constexpr int kNormPollers = 256;  // threads that poll, for one or two workgroups each
+constexpr int kNormMaxBlocks = 2 * kNormPollers;
 constexpr int kNormFirst = 8, kNormStates = kNormFirst + kNormWords * kNormMaxBlocks;
 constexpr int kNormSyncWords = kNormStates + kNormMaxBlocks;
 constexpr uint32_t kNormMaxEpoch = 0xffff;
@@ -855,13 +856,13 @@ struct in_one_launch<OneLaunchOp<StatsOp>> : std::true_type {};
 // st: the thread's statistics.  store(f): stores f(advantage) for every advantage the thread
 // holds (E rounds to the storage type as the raw store of two launches would).  region(j, first,
 // count): where workgroup j's advantages lie in x.  Called by every thread, at least
-// kNormMaxBlocks of them.
+// kNormPollers of them.
 template <int NT, class E, class Store, class Region>
 __device__ __forceinline__ void finish_normalized(const OneLaunch& one, Stats st, E* __restrict__ x, int waves,
                                                   Store store, Region region) {
-  constexpr int NW = NT / kWave, PW = kNormMaxBlocks / kWave;
+  constexpr int NW = NT / kWave, PW = kNormPollers / kWave;
   constexpr uint64_t kLow48 = (uint64_t{1} << 48) - 1;
-  static_assert(NW >= PW, "a thread per workgroup");
+  static_assert(NW >= PW, "threads that poll");
   __shared__ double s_own[kStatWords][NW], s_all[kStatWords][PW];
   __shared__ int s_seen[PW];
   __shared__ int s_claimed[kNormMaxBlocks];
@@ -888,31 +889,44 @@ __device__ __forceinline__ void finish_normalized(const OneLaunch& one, Stats st
     const uint64_t high = lane_u64<0>(u) >> 48 | lane_u64<1>(u) >> 48 << 16 | lane_u64<2>(u) >> 48 << 32;
     if (lane < kNormWords) atomic_st(line(own) + lane, tag | (lane < kStatWords ? u & kLow48 : high));
   }
-  // All statistics into s_all; false if some are missing after `polls` more reads.
-  auto gather = [&](int polls) -> bool {
+  // All statistics into s_all; false if some are missing after `polls` more reads.  R: workgroups
+  // per polling thread.
+  auto gather_r = [&](int polls, auto r_const) -> bool {
+    constexpr int R = decltype(r_const)::value;
     if (wave < PW) {
-      uint64_t v[kNormWords];
-      bool here = tid >= nb;
+      uint64_t v[R][kNormWords];
+      bool here[R];
+#pragma unroll
+      for (int r = 0; r < R; ++r) here[r] = tid + r * kNormPollers >= nb;
+      bool all = false;
       for (int p = 0;; ++p) {
-        if (!here) {
+        all = true;
 #pragma unroll
-          for (int i = 0; i < kNormWords; ++i) v[i] = atomic_ld(line(tid) + i);
-          here = true;
+        for (int r = 0; r < R; ++r) {
+          if (!here[r]) {
 #pragma unroll
-          for (int i = 0; i < kNormWords; ++i) here = here && (v[i] & ~kLow48) == tag;
+            for (int i = 0; i < kNormWords; ++i) v[r][i] = atomic_ld(line(tid + r * kNormPollers) + i);
+            here[r] = true;
+#pragma unroll
+            for (int i = 0; i < kNormWords; ++i) here[r] = here[r] && (v[r][i] & ~kLow48) == tag;
+          }
+          all = all && here[r];
         }
-        if (__ballot(!here) == 0 || p >= polls) break;
+        if (__ballot(!all) == 0 || p >= polls) break;
         __builtin_amdgcn_s_sleep(1);
       }
-      const bool seen = __ballot(!here) == 0;
+      const bool seen = __ballot(!all) == 0;
       wait_vmem();  // wave 0: this workgroup's statistics are visible
       asm volatile("" : : : "memory");
       if (lane == 0) s_seen[wave] = seen;
 #pragma unroll
       for (int k = 0; k < kStatWords; ++k) {
         double a = 0.0;
-        if (seen && tid < nb)
-          a += __longlong_as_double((long long)((v[k] & kLow48) | (v[kNormWords - 1] >> (16 * k)) << 48));
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+          if (seen && tid + r * kNormPollers < nb)
+            a += __longlong_as_double((long long)((v[r][k] & kLow48) | (v[r][kNormWords - 1] >> (16 * k)) << 48));
+        }
         a = wave_total(a);
         if (lane == kWave - 1) s_all[k][wave] = a;
       }
@@ -922,6 +936,10 @@ __device__ __forceinline__ void finish_normalized(const OneLaunch& one, Stats st
 #pragma unroll
     for (int w = 0; w < PW; ++w) seen = seen && s_seen[w] != 0;
     return seen;
+  };
+  auto gather = [&](int polls) -> bool {
+    return nb <= kNormPollers ? gather_r(polls, std::integral_constant<int, 1>{})
+                              : gather_r(polls, std::integral_constant<int, 2>{});
   };
   auto totals = [&](float& m, float& d) {
     double t[kStatWords] = {0.0, 0.0, 0.0};
@@ -968,12 +986,12 @@ __device__ __forceinline__ void finish_normalized(const OneLaunch& one, Stats st
   __syncthreads();
   if (tid == 0) s_nclaimed = 0;
   __syncthreads();
-  if (tid < nb) {
+  for (int j = tid; j < nb; j += blockDim.x) {
     uint64_t raw = tag | kNormRaw;
-    if (atomic_ld(state + tid) == raw &&
-        __hip_atomic_compare_exchange_strong(state + tid, &raw, tag | kNormClaimed, __ATOMIC_ACQ_REL,
+    if (atomic_ld(state + j) == raw &&
+        __hip_atomic_compare_exchange_strong(state + j, &raw, tag | kNormClaimed, __ATOMIC_ACQ_REL,
                                              __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
-      s_claimed[atomicAdd(&s_nclaimed, 1)] = tid;
+      s_claimed[atomicAdd(&s_nclaimed, 1)] = j;
   }
   __syncthreads();
   const int claimed = s_nclaimed;

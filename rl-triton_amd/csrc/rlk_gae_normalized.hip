@@ -109,7 +109,7 @@ extern "C" {
 
 int rlk_gae_normalized_one_launch_takes(int64_t num_envs, int64_t seq_len) {
   // A workgroup holds at most 4096 advantages of short rows, or one whole longer row.
-  if (seq_len <= kShortMaxT) return num_envs * seq_len <= (int64_t)kNormMaxBlocks * 4096;
+  if (seq_len <= kShortMaxT) return num_envs * seq_len <= (int64_t)kNormPollers * 4096;
   return num_envs <= kNormMaxBlocks && whole_row_segments<GaeStatsOp<true>>(num_envs, seq_len, true) > 0;
 }
 

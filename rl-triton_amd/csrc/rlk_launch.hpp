@@ -330,13 +330,13 @@ struct paired_rows : std::false_type {};
 template <int NA, bool TRUNC>
 struct paired_rows<RetraceOp<NA, TRUNC, float>> : std::bool_constant<(NA > 0)> {};
 
-// Whether a launch's workgroups all fit the GPU at once (for the normalisation in the scan's own
-// launch; a wrong answer costs time, not results).  The runtime's answer per kernel and
+// Whether a launch is one for the normalisation in the scan's own launch: at most `most`
+// workgroups that all fit the GPU at once (a wrong answer costs time, not results).  The runtime's answer per kernel and
 // workgroup size is kept.
-inline bool all_resident(const void* kernel, int64_t blocks, int threads, size_t lds) {
+inline bool all_resident(const void* kernel, int64_t blocks, int64_t most, int threads, size_t lds) {
   static std::mutex mu;
   static std::map<std::pair<const void*, int>, int> per_cu;
-  if (blocks > kNormMaxBlocks || threads < kNormMaxBlocks) return false;
+  if (blocks > most || threads < kNormPollers) return false;
   std::lock_guard<std::mutex> lock(mu);
   auto it = per_cu.find({kernel, threads});
   if (it == per_cu.end()) {
@@ -347,13 +347,18 @@ inline bool all_resident(const void* kernel, int64_t blocks, int threads, size_t
   return blocks <= (int64_t)it->second * device_cus();
 }
 
-// A kernel launch of an op.  hipErrorNotReady, and nothing launched: a OneLaunchOp's workgroups do
-// not fit at once.
+// A kernel launch of an op.  hipErrorNotReady, and nothing launched: a OneLaunchOp with more than
+// one_launch_blocks workgroups, or more than fit at once.  Beyond kNormPollers workgroups the
+// exchange costs more than a second launch for rows of up to 1024 steps ([6000,128] 8.5 -> 9.5 us,
+// [2000,300] 8.0 -> 10.3, [1024,1000] 9.5 -> 11.1), and less where each workgroup holds a row of
+// more (kNormMaxBlocks; [512,2048] 9.5 -> 8.9, [512,4096] 16.0 -> 13.8, masked [512,6000]
+// 22.5 -> 19.1, [512,8192] 25.8 -> 22.0).
 template <class Op>
-hipError_t launch_kernel(const void* kernel, const Op& op, int64_t blocks, int threads, void** args, hipStream_t stream) {
+hipError_t launch_kernel(const void* kernel, const Op& op, int64_t blocks, int threads, void** args, hipStream_t stream,
+                         int64_t one_launch_blocks = kNormPollers) {
   const size_t lds = dynamic_lds(op, threads);
   if constexpr (in_one_launch<Op>::value) {
-    if (!all_resident(kernel, blocks, threads, lds)) return hipErrorNotReady;
+    if (!all_resident(kernel, blocks, one_launch_blocks, threads, lds)) return hipErrorNotReady;
   }
   return hipLaunchKernel(kernel, dim3((unsigned)blocks), dim3(threads), args, lds, stream);
 }
@@ -403,7 +408,7 @@ hipError_t launch_strided(const Op& op, int64_t E, int T, int threads, hipStream
   int unused = 0;
   void* args[] = {const_cast<Op*>(&op), &E, &T, &unused};
   return launch_kernel(reinterpret_cast<const void*>(&rows_strided_kernel<Op, NT, Q, VEC, 1>), op, E, threads, args,
-                       stream);
+                       stream, kNormMaxBlocks);
 }
 
 template <class Op, int VEC>
