@@ -17,8 +17,8 @@
  *     default stream).  Nothing allocates and nothing synchronises.
  *   - Any element-aligned pointers are accepted.  The fastest form is seq_len % 4 == 0
  *     with every [num_envs, seq_len] array 16-byte aligned (bfloat16: 8-byte), which
- *     the kernels read and write with aligned non-temporal 16-byte accesses.  Rows longer
- *     than 2048 steps of seq_len % 4 != 0 whose arrays all start at the same element
+ *     the kernels read and write with aligned non-temporal 16-byte accesses.  Rows split
+ *     into tiles, of seq_len % 4 != 0, whose arrays all start at the same element
  *     offset modulo 4 (freshly allocated arrays do) are shifted to their own 16-byte
  *     boundaries and keep aligned accesses (within ~5% of the aligned form); Retrace and
  *     the normalised GAE entries excepted.  Other calls use element-aligned 16-byte
@@ -27,7 +27,7 @@
  *     (bootstrap is [num_envs]: the continuation value after step seq_len-1, the
  *     reference's `last_value`), RLK_BOOT_FULL (bootstrap is [num_envs, seq_len], the
  *     reference's `bootstrap_values`).
- *   - Workspace: rows longer than one workgroup tile are split into tiles chained by a
+ *   - Workspace: rows of more than 2048 steps can be split into tiles chained by a
  *     decoupled look-back.  Those calls need `workspace` of at least
  *     rlk_workspace_bytes(num_envs, seq_len) bytes, ZERO-FILLED BEFORE ITS FIRST USE.
  *     Each call leaves the workspace ready for the next one, so zero it once and reuse

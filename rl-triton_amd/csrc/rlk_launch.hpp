@@ -186,6 +186,8 @@ inline int64_t tile_steps(LongShape s) { return (int64_t)s.threads * kSeg * s.se
 //     look-back chain along a row, so a call of many rows of a few thousand steps ran one
 //     tile per row that was mostly padding: a 2560-step row in a 32768-step tile, the
 //     prefix sum [4096,2560] at 114 us against 22 us for a streaming kernel of its bytes.
+//     (Such rows are now held whole, see whole_row_segments; this serves longer ones and
+//     Retrace's.)
 //     Where more than a quarter of a row's tile steps would be padding, the call takes the
 //     largest of the op's tiles that pads a row by at most a quarter, or else the one that
 //     pads it least (the larger on a tie), unless its tiles fit the CUs in one round and
