@@ -10,7 +10,8 @@ replaces is what a PPO loop writes after compute_gae:
 
 Here the scan writes the raw advantages, the returns and per-workgroup float64 partial sums
 in one pass; a second launch turns the advantages into (A - mean) / (std + eps) in place
-(std unbiased, as Tensor.std()).  The statistics are reduced in a fixed order, so results
+(std unbiased, as Tensor.std()).  Where all workgroups fit the GPU at once, one launch does
+both and the raw advantages stay in registers.  The statistics are reduced in a fixed order, so results
 are bit-reproducible run to run.
 """
 import torch
