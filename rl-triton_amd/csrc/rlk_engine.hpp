@@ -546,6 +546,14 @@ __device__ __forceinline__ uint64_t pack(uint32_t tag, float v) {
 // its path rejoins the other waves', so nothing it issued looks pending to the compiler.)
 __device__ __forceinline__ void wait_vmem() { __builtin_amdgcn_s_waitcnt(0x0F70); }
 
+// __threadfence() for what the thread stored by inline assembly too (store_quad_wt): the compiler
+// does not count those stores as pending, and drops the fence's wait where nothing else is.
+__device__ __forceinline__ void threadfence_all_stores() {
+  wait_vmem();
+  __threadfence();
+  wait_vmem();
+}
+
 // Lane L's value of a 64-bit register, in every lane.
 template <int L>
 __device__ __forceinline__ uint64_t lane_u64(uint64_t x) {
@@ -955,7 +963,7 @@ __device__ __forceinline__ void finish_normalized(const OneLaunch& one, Stats st
   uint64_t look = 0;  // the "some workgroup is raw" word, read once what this workgroup published is visible
   if (!gather(one.polls)) {
     store([](float a) { return a; });
-    __threadfence();
+    threadfence_all_stores();
     __syncthreads();
     if (tid == 0) {
       atomic_st(state + own, tag | kNormRaw);

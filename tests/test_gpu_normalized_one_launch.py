@@ -96,3 +96,19 @@ def test_streams_and_call_limit(device, monkeypatch):
                 assert torch.equal(g, w)
     finally:
         _native.fast.set_workspace_max_calls(prev)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["f32", "bf16"])
+@pytest.mark.parametrize("trunc", [False, True])
+@pytest.mark.parametrize("masked", [False, True])
+@pytest.mark.parametrize("shape", [(200, 9000), (130, 9217)], ids=lambda s: f"{s[0]}x{s[1]}")
+def test_four_segment_rows(shape, masked, trunc, dtype, polls, device):
+    """Four segments per thread, with and without truncations (instances of their own): a workgroup
+    that stops waiting marks its raw advantages only once they are written."""
+    op = "gae_normalized_masked" if masked else "gae_normalized"
+    inp, params = make_inputs(op, *shape, seed=sum(shape), p_trunc=0.02 if trunc else 0.0, boot="full" if trunc else "row")
+    d = to_device(inp, device, dtype)
+    want = _two_launches(d, params)
+    for _ in range(5):
+        for g, w in zip(_call(d, params), want):
+            assert torch.equal(g.view(torch.int16), w.view(torch.int16)), f"{op}{shape} {dtype}"
