@@ -1350,23 +1350,40 @@ __device__ __forceinline__ typename M::State tile_carry(M tm, typename M::State 
   const uint64_t* sf = fb + NWD * (row * (int64_t)tiles_per_row);
   const uint32_t tag_agg = (epoch << 2) | kAgg, tag_inc = (epoch << 2) | kInc;
   need = -1;
+  // Every tile along a row waits for the publishes before it in turn, so they are kept short.  In
+  // backward scans the tile's own words have one address: formed at each publish, under branches
+  // that tell the compiler more of k, it was three values, two of them spilled and reloaded right
+  // there; and each publish ends in an assembly comment of its own, or the compiler joins their
+  // last stores behind one more branch.  (Discounted returns [37,20011] 5.40 -> 5.35 us, V-trace
+  // [16,131072] 11.77 -> 11.6 on most GPUs.  Forward scans have no such spills: one address added
+  // a spill to the 32768-step instances, prefix sum [8,2^20] 18.09 -> 18.16.)
+  uint64_t* const own_words = st + NWD * k;
+  auto own = [&]() -> uint64_t* {
+    if constexpr (FWD) return st + NWD * k;
+    else return own_words;
+  };
   // word 0 last: it names the kind
   auto publish_inc = [&](State x) {
 #pragma unroll
-    for (int i = NSW - 1; i >= 0; --i) atomic_st(st + NWD * k + i, pack(tag_inc, state_word(x, i)));
+    for (int i = NSW - 1; i >= 0; --i) atomic_st(own() + i, pack(tag_inc, state_word(x, i)));
   };
   if (FWD ? (k == 0) : (k == tiles_per_row - 1)) {
     wait_vmem();
-    if (lane == 0) publish_inc(tm.apply(row_c));
+    if (lane == 0) {
+      publish_inc(tm.apply(row_c));
+      if constexpr (!FWD) asm volatile("; the row's first tile");
+    }
     return row_c;
   }
   if (lane == 0) {
     if (tm.constant()) {
       // the tile's outgoing state does not depend on its carry
       publish_inc(tm.apply(State{}));
+      if constexpr (!FWD) asm volatile("; a constant map");
     } else {
 #pragma unroll
-      for (int i = NWD - 1; i >= 0; --i) atomic_st(st + NWD * k + i, pack(tag_agg, tm.word(i)));
+      for (int i = NWD - 1; i >= 0; --i) atomic_st(own() + i, pack(tag_agg, tm.word(i)));
+      if constexpr (!FWD) asm volatile("; a map");
     }
   }
   auto tile_at = [&](int base, int l) { return FWD ? k - 1 - base - l : k + 1 + base + l; };
@@ -1454,7 +1471,10 @@ __device__ __forceinline__ typename M::State tile_carry(M tm, typename M::State 
     c = nan_state<State>();
   }
   wait_vmem();
-  if (lane == 0 && !tm.constant()) publish_inc(tm.apply(c));
+  if (lane == 0 && !tm.constant()) {
+    publish_inc(tm.apply(c));
+    if constexpr (!FWD) asm volatile("; a state");
+  }
   return c;
 }
 
