@@ -333,12 +333,18 @@ template <int NA, bool TRUNC>
 struct paired_rows<RetraceOp<NA, TRUNC, float>> : std::bool_constant<(NA > 0)> {};
 
 // Whether a launch is one for the normalisation in the scan's own launch: at most `most`
-// workgroups that all fit the GPU at once (a wrong answer costs time, not results).  The runtime's answer per kernel and
-// workgroup size is kept.
+// workgroups that all fit the GPU at once (a wrong answer costs time, not results, but much of it:
+// the workgroups that are resident wait out their polls).  The runtime's answer per kernel and
+// workgroup size is kept.  It is asked for whole fours of waves: a CU deals a workgroup's waves to
+// its four SIMDs, so one of 14 takes four wave slots of the fullest, and two of them do not fit
+// SIMDs of seven slots, of which the runtime counts 28 (72-register masked kernels, [300,7000]:
+// 350 us in one launch, 23 in two).
 inline bool all_resident(const void* kernel, int64_t blocks, int64_t most, int threads, size_t lds) {
   static std::mutex mu;
   static std::map<std::pair<const void*, int>, int> per_cu;
   if (blocks > most || threads < kNormPollers) return false;
+  constexpr int kSimdWaves = 4 * kWave;
+  threads = (threads + kSimdWaves - 1) / kSimdWaves * kSimdWaves;
   std::lock_guard<std::mutex> lock(mu);
   auto it = per_cu.find({kernel, threads});
   if (it == per_cu.end()) {

@@ -257,6 +257,7 @@ int dispatch(const Call& c, Body body) {
 
 // Calls this module has launched (a diagnostic for tests: which path served a call).
 uint64_t g_launched = 0;
+uint64_t g_one_launches = 0;
 
 PyObject* finish(int status, const char* what, PyObject* result) {
   ++g_launched;
@@ -380,7 +381,10 @@ PyObject* op_gae_normalized(PyObject* const* a, Py_ssize_t n) {
     if (ask_one_launch(c, *r, t)) {
       t.out[0] = adv.data_ptr(), t.out[1] = ret.data_ptr();
       const int st = rlk_time_major(&t, c.stream());
-      if (st <= 0) return finish(st, "rlk_time_major", pair(adv, ret));
+      if (st <= 0) {
+        ++g_one_launches;
+        return finish(st, "rlk_time_major", pair(adv, ret));
+      }
       t.sync = nullptr;
     }
     t.partials_bytes = rlk_time_major_partials_bytes(c.E, c.T);
@@ -396,7 +400,10 @@ PyObject* op_gae_normalized(PyObject* const* a, Py_ssize_t n) {
     t.out[0] = adv.data_ptr(), t.out[1] = ret.data_ptr();
     if (ask_one_launch(c, *r, t)) {
       const int st = rlk_gae_normalized_one_launch(&t, c.stream());
-      if (st <= 0) return finish(st, "rlk_gae_normalized_one_launch", pair(adv, ret));
+      if (st <= 0) {
+        ++g_one_launches;
+        return finish(st, "rlk_gae_normalized_one_launch", pair(adv, ret));
+      }
     }
   }
   const Workspace ws = workspace(c, *r);
@@ -857,6 +864,27 @@ PyObject* set_workspace_max_calls(PyObject*, PyObject* arg) {
   return PyLong_FromUnsignedLongLong(prev);
 }
 
+// norm_syncs() -> [(device, epoch, buffer)] of normalised GAE in one launch, in order of device and
+// stream (a diagnostic for tests: which form served a call, and how it ended).
+PyObject* norm_syncs_list(PyObject*, PyObject*) {
+  PyObject* out = PyList_New(0);
+  if (!out) return nullptr;
+  for (auto& kv : norm_syncs()) {
+    if (!kv.second.buf.defined()) continue;
+    PyObject* t = Py_BuildValue("(iIN)", kv.first.first, kv.second.epoch, THPVariable_Wrap(kv.second.buf));
+    if (!t || PyList_Append(out, t) != 0) {
+      Py_XDECREF(t);
+      Py_DECREF(out);
+      return nullptr;
+    }
+    Py_DECREF(t);
+  }
+  return out;
+}
+
+// Normalised GAE calls served in one launch (a diagnostic for tests).
+PyObject* one_launches(PyObject*, PyObject*) { return PyLong_FromUnsignedLongLong(g_one_launches); }
+
 PyObject* workspace_clears(PyObject*, PyObject*) { return PyLong_FromUnsignedLongLong(g_ws_clears); }
 
 PyMethodDef kMethods[] = {
@@ -866,6 +894,10 @@ PyMethodDef kMethods[] = {
      "cached workspace (n <= 0: the default, RLK_WORKSPACE_MAX_CALLS)"},
     {"workspace_clears", workspace_clears, METH_NOARGS,
      "workspace_clears() -> cached workspaces zero-filled again at the call limit so far"},
+    {"norm_syncs", norm_syncs_list, METH_NOARGS,
+     "norm_syncs() -> [(device, epoch, buffer)] of normalised GAE calls in one launch"},
+    {"one_launches", one_launches, METH_NOARGS,
+     "one_launches() -> normalised GAE calls the fast path has served in one launch so far"},
     {"launched", launched, METH_NOARGS, "launched() -> calls the fast path has launched so far"},
     {"workspace_error", workspace_error, METH_O,
      "workspace_error(device) -> True if a look-back wait of this module's calls gave up"},

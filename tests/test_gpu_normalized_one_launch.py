@@ -112,3 +112,71 @@ def test_four_segment_rows(shape, masked, trunc, dtype, polls, device):
     for _ in range(5):
         for g, w in zip(_call(d, params), want):
             assert torch.equal(g.view(torch.int16), w.view(torch.int16)), f"{op}{shape} {dtype}"
+
+
+def _marks():
+    """How many workgroups of the last one-launch call on each stream stopped waiting: words of the
+    buffer's state part (behind 8 words and 4 per workgroup, 512 workgroups) with that call's epoch,
+    marked raw (1) or raw and normalised by another workgroup (2)."""
+    from rl_triton import _native
+    raw = claimed = 0
+    for _, epoch, buf in _native.fast.norm_syncs():
+        state = buf.view(torch.int64)[8 + 4 * 512:].cpu()
+        assert state.numel() == 512
+        mine = state[(state >> 48) & 0xffff == epoch] & 0xffff
+        raw, claimed = raw + int((mine == 1).sum()), claimed + int((mine == 2).sum())
+    return raw, claimed
+
+
+def _one_launches():
+    from rl_triton import _native
+    return _native.fast.one_launches()
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["f32", "bf16"])
+@pytest.mark.parametrize("masked", [False, True])
+@pytest.mark.parametrize("shape", [(64, 64), (1024, 128), (256, 2048), (300, 1100), (512, 2052), (512, 6000), (257, 6148),
+                                   (300, 6656), (300, 6660), (300, 7000), (512, 7168), (257, 7172), (300, 8192),
+                                   (256, 9000), (256, 16384)], ids=lambda s: f"{s[0]}x{s[1]}")
+def test_no_workgroup_stops_waiting(shape, masked, dtype, device, monkeypatch):
+    """A call takes one launch only where its workgroups are resident together: with nothing else on
+    the GPU none of them runs out of polls.  (Twelve waves of four segments per thread and more are
+    where a CU's register count and its SIMDs' wave slots differ.)"""
+    monkeypatch.delenv("RL_TRITON_CORRECTNESS_WARNINGS", raising=False)
+    op = "gae_normalized_masked" if masked else "gae_normalized"
+    inp, params = make_inputs(op, *shape, seed=1, boot="row")
+    d = to_device(inp, device, dtype)
+    for _ in range(3):
+        torch.cuda.synchronize()
+        _call(d, params)
+        torch.cuda.synchronize()
+        assert _marks() == (0, 0)
+
+
+@pytest.mark.parametrize("masked", [False, True])
+@pytest.mark.parametrize("shape", [(1024, 128), (256, 4096), (200, 9000), (130, 9217)], ids=lambda s: f"{s[0]}x{s[1]}")
+def test_raw_advantages_are_claimed_once(shape, masked, device, monkeypatch):
+    """Workgroups that never look again stop waiting, unless all others came first: each one marked
+    raw is taken by one that has all statistics, and none is left."""
+    from rl_triton import _native
+    monkeypatch.delenv("RL_TRITON_CORRECTNESS_WARNINGS", raising=False)
+    op = "gae_normalized_masked" if masked else "gae_normalized"
+    inp, params = make_inputs(op, *shape, seed=2, boot="row")
+    d = to_device(inp, device)
+    want = _two_launches(d, params)
+    _native.load().rlk_debug_lookback(-1, 0)
+    try:
+        claimed = 0
+        for _ in range(5):
+            before = _one_launches()
+            got = _call(d, params)
+            torch.cuda.synchronize()
+            assert _one_launches() == before + 1
+            raw, c = _marks()
+            claimed += c
+            assert raw == 0
+            for g, w in zip(got, want):
+                assert torch.equal(g, w)
+        assert claimed > 0
+    finally:
+        _native.load().rlk_debug_lookback(-1, -1)
