@@ -65,8 +65,9 @@ int rlk_time_major(const rlk_time_major_call *call, void *stream);
 #define RLK_NORM_SYNC_BYTES (8 * (8 + 4 * 512 + 512))
 #define RLK_NORM_MAX_EPOCH 0xffff
 int rlk_gae_normalized_one_launch(const rlk_time_major_call *call, void *stream);
-/* 0: no call of this shape takes one launch (a quick look, in either layout). */
-int rlk_gae_normalized_one_launch_takes(int64_t num_envs, int64_t seq_len);
+/* 0: no call of this shape takes one launch (contiguous rows; time-major). */
+int rlk_gae_normalized_one_launch_takes(int64_t num_envs, int64_t seq_len, int masked);
+int rlk_time_major_one_launch_takes(int64_t num_envs, int64_t seq_len);
 
 #ifdef __cplusplus
 }

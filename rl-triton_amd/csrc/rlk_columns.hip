@@ -149,6 +149,11 @@ int rlk_time_major_takes(int64_t num_envs, int64_t seq_len, int64_t step_stride,
   return takes(num_envs, seq_len, step_stride, num_actions) ? 1 : 0;
 }
 
+int rlk_time_major_one_launch_takes(int64_t num_envs, int64_t seq_len) {
+  if (num_envs <= 0 || seq_len <= 0 || seq_len > 4 * kWave / kCols * column_waves<GaeStatsOp<true>>::value) return 0;
+  return column_blocks<GaeStatsOp<true>>(num_envs, seq_len) <= kNormPollers ? 1 : 0;
+}
+
 size_t rlk_time_major_partials_bytes(int64_t num_envs, int64_t seq_len) {
   if (num_envs <= 0 || seq_len <= 0) return 0;
   return (size_t)partials_triples(column_blocks<GaeStatsOp<true>>(num_envs, seq_len)) * kStatWords * sizeof(double);

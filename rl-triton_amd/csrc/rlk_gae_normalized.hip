@@ -107,10 +107,18 @@ using namespace rlk;
 
 extern "C" {
 
-int rlk_gae_normalized_one_launch_takes(int64_t num_envs, int64_t seq_len) {
-  // A workgroup holds at most 4096 advantages of short rows, or one whole longer row.
-  if (seq_len <= kShortMaxT) return num_envs * seq_len <= (int64_t)kNormPollers * 4096;
-  return num_envs <= kNormMaxBlocks && whole_row_segments<GaeStatsOp<true>>(num_envs, seq_len, true) > 0;
+int rlk_gae_normalized_one_launch_takes(int64_t num_envs, int64_t seq_len, int masked) {
+  // Asked ahead of every call: one that launch() then refused would pay for both forms on the host
+  // ([1000,500] 8.1 us per call, 7.8 so).
+  const int64_t E = num_envs, T = seq_len;
+  if (E <= 0 || T <= 0 || T > 4 * kWholeRowThreads * kSeg) return 0;
+  const int64_t most = T > kShortMaxT || T % 4 == 0 ? one_launch_blocks(T, masked != 0) : kNormPollers;
+  if (T > kShortMaxT / 2)  // a workgroup per row
+    return E <= most && (T <= kShortMaxT || whole_row_segments<GaeStatsOp<true>>(E, T, true) > 0) ? 1 : 0;
+  // the finest grid, the coarsest, else the one it is
+  if (rows_grid(E, T, rows_seg(T), kNT) <= most) return 1;
+  if (rows_grid(E, T, rows_seg(T), kNTWide) > most) return 0;
+  return launch_grid<GaeStatsOp<true>>(E, T) <= most ? 1 : 0;
 }
 
 int rlk_gae_normalized_one_launch(const rlk_time_major_call* call, void* stream) {

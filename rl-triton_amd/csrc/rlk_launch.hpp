@@ -355,18 +355,30 @@ inline bool all_resident(const void* kernel, int64_t blocks, int64_t most, int t
   return blocks <= (int64_t)it->second * device_cus();
 }
 
+// Most workgroups of a normalised GAE in one launch.  Beyond kNormPollers the exchange costs more
+// than a second launch for rows of up to 1024 steps ([6000,128] 8.5 -> 9.5 us, [2000,300] 8.0 ->
+// 10.3, [1024,1000] 9.5 -> 11.1), and less where each workgroup holds a longer row: kNormMaxBlocks
+// ([512,2048] 9.5 -> 8.9, [512,4096] 16.0 -> 13.8, masked [512,6000] 22.5 -> 19.1, [512,8192]
+// 25.8 -> 22.0), for masked rows of up to 2048 steps kNormMaskedBlocks (one launch over two at 300
+// rows 0.89-0.96, at 384 0.97-1.03, at 448 1.02-1.07, at 512 1.02-1.08).
+constexpr int64_t kNormMaskedBlocks = 384;
+inline int64_t one_launch_blocks(int64_t T, bool masked) {
+  if (T <= kShortMaxT / 2) return kNormPollers;
+  return masked && T <= kShortMaxT ? kNormMaskedBlocks : kNormMaxBlocks;
+}
+template <class Op>
+struct masked_stats : std::false_type {};
+template <bool TRUNC, class E>
+struct masked_stats<OneLaunchOp<MaskedGaeStatsOp<TRUNC, E>>> : std::true_type {};
+
 // A kernel launch of an op.  hipErrorNotReady, and nothing launched: a OneLaunchOp with more than
-// one_launch_blocks workgroups, or more than fit at once.  Beyond kNormPollers workgroups the
-// exchange costs more than a second launch for rows of up to 1024 steps ([6000,128] 8.5 -> 9.5 us,
-// [2000,300] 8.0 -> 10.3, [1024,1000] 9.5 -> 11.1), and less where each workgroup holds a row of
-// more (kNormMaxBlocks; [512,2048] 9.5 -> 8.9, [512,4096] 16.0 -> 13.8, masked [512,6000]
-// 22.5 -> 19.1, [512,8192] 25.8 -> 22.0).
+// `most` workgroups, or more than fit at once.
 template <class Op>
 hipError_t launch_kernel(const void* kernel, const Op& op, int64_t blocks, int threads, void** args, hipStream_t stream,
-                         int64_t one_launch_blocks = kNormPollers) {
+                         int64_t most = kNormPollers) {
   const size_t lds = dynamic_lds(op, threads);
   if constexpr (in_one_launch<Op>::value) {
-    if (!all_resident(kernel, blocks, one_launch_blocks, threads, lds)) return hipErrorNotReady;
+    if (!all_resident(kernel, blocks, most, threads, lds)) return hipErrorNotReady;
   }
   return hipLaunchKernel(kernel, dim3((unsigned)blocks), dim3(threads), args, lds, stream);
 }
@@ -416,7 +428,7 @@ hipError_t launch_strided(const Op& op, int64_t E, int T, int threads, hipStream
   int unused = 0;
   void* args[] = {const_cast<Op*>(&op), &E, &T, &unused};
   return launch_kernel(reinterpret_cast<const void*>(&rows_strided_kernel<Op, NT, Q, VEC, 1>), op, E, threads, args,
-                       stream, kNormMaxBlocks);
+                       stream, one_launch_blocks(T, masked_stats<Op>::value));
 }
 
 template <class Op, int VEC>

@@ -213,10 +213,15 @@ std::map<std::pair<int, uintptr_t>, NormSync>& norm_syncs() {
   return *m;
 }
 
-// Asks for one launch: false for shapes that never take it and while the stream is capturing a
-// graph, whose replays would repeat the epoch.
+// Whether calls of this shape take one launch.
+bool one_launch_shape(const Call& c, bool masked) {
+  return (c.ld > 0 ? rlk_time_major_one_launch_takes(c.E, c.T)
+                   : rlk_gae_normalized_one_launch_takes(c.E, c.T, masked)) != 0;
+}
+
+// Asks for one launch: false while the stream is capturing a graph, whose replays would repeat the
+// epoch.
 bool ask_one_launch(const Call& c, const at::Tensor& like, rlk_time_major_call& t) {
-  if (!rlk_gae_normalized_one_launch_takes(c.E, c.T)) return false;
   hipStream_t s = static_cast<hipStream_t>(c.stream());
   hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
   if (hipStreamIsCapturing(s, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone) return false;
@@ -378,7 +383,7 @@ PyObject* op_gae_normalized(PyObject* const* a, Py_ssize_t n) {
     rlk_time_major_call t = time_major(c, RLK_OP_GAE_NORMALIZED, in, 5, boot, mode);
     t.gamma = gamma, t.lambda_ = lam, t.eps = eps;
     at::Tensor adv = c.output(*r), ret = c.output(*r);
-    if (ask_one_launch(c, *r, t)) {
+    if (one_launch_shape(c, mask != nullptr) && ask_one_launch(c, *r, t)) {
       t.out[0] = adv.data_ptr(), t.out[1] = ret.data_ptr();
       const int st = rlk_time_major(&t, c.stream());
       if (st <= 0) {
@@ -393,7 +398,7 @@ PyObject* op_gae_normalized(PyObject* const* a, Py_ssize_t n) {
     return finish(rlk_time_major(&t, c.stream()), "rlk_time_major", pair(adv, ret));
   }
   at::Tensor adv = c.output(*r), ret = c.output(*r);
-  {
+  if (one_launch_shape(c, mask != nullptr)) {
     const at::Tensor* in[] = {r, v, te, tr, mask};
     rlk_time_major_call t = time_major(c, RLK_OP_GAE_NORMALIZED, in, 5, boot, mode);
     t.gamma = gamma, t.lambda_ = lam, t.eps = eps;

@@ -137,7 +137,7 @@ def _one_launches():
 @pytest.mark.parametrize("masked", [False, True])
 @pytest.mark.parametrize("shape", [(64, 64), (1024, 128), (256, 2048), (300, 1100), (512, 2052), (512, 6000), (257, 6148),
                                    (300, 6656), (300, 6660), (300, 7000), (512, 7168), (257, 7172), (300, 8192),
-                                   (256, 9000), (256, 16384)], ids=lambda s: f"{s[0]}x{s[1]}")
+                                   (256, 9000), (400, 9000), (300, 12000), (256, 16384)], ids=lambda s: f"{s[0]}x{s[1]}")
 def test_no_workgroup_stops_waiting(shape, masked, dtype, device, monkeypatch):
     """A call takes one launch only where its workgroups are resident together: with nothing else on
     the GPU none of them runs out of polls.  (Twelve waves of four segments per thread and more are
@@ -180,3 +180,34 @@ def test_raw_advantages_are_claimed_once(shape, masked, device, monkeypatch):
         assert claimed > 0
     finally:
         _native.load().rlk_debug_lookback(-1, -1)
+
+
+# (shape, one launch unmasked, one launch masked): both sides of each line of one_launch_blocks
+@pytest.mark.parametrize("shape,plain,masked", [
+    ((64, 64), True, True), ((4096, 128), True, True), ((4097, 128), False, False), ((256, 1024), True, True),
+    ((1024, 1000), False, False), ((384, 1028), True, True), ((385, 1028), True, False), ((512, 2048), True, False),
+    ((513, 2048), False, False), ((256, 2047), True, True), ((257, 2047), False, False), ((512, 2049), True, True),
+    ((513, 2049), False, False), ((512, 6000), True, True), ((300, 7000), True, False), ((512, 8192), True, False),
+    ((256, 9000), True, True), ((257, 9000), True, False), ((3, 16385), False, False)],
+    ids=lambda s: f"{s[0]}x{s[1]}" if isinstance(s, tuple) else None)
+def test_which_calls_take_one_launch(shape, plain, masked, device, monkeypatch):
+    monkeypatch.delenv("RL_TRITON_CORRECTNESS_WARNINGS", raising=False)
+    for op, want in (("gae_normalized", plain), ("gae_normalized_masked", masked)):
+        inp, params = make_inputs(op, *shape, seed=4, boot="row")
+        d = to_device(inp, device)
+        before = _one_launches()
+        _call(d, params)
+        assert _one_launches() - before == want, op
+        before = _one_launches()
+        _two_launches(d, params)
+        assert _one_launches() - before == want, f"{op}: a captured call"
+
+
+@pytest.mark.parametrize("shape,want", [((64, 64), True), ((4096, 128), True), ((4112, 128), False), ((100, 256), True),
+                                        ((100, 257), False)], ids=lambda s: f"{s[0]}x{s[1]}" if isinstance(s, tuple) else None)
+def test_which_time_major_calls_take_one_launch(shape, want, device, monkeypatch):
+    monkeypatch.delenv("RL_TRITON_CORRECTNESS_WARNINGS", raising=False)
+    inp, params = make_inputs("gae_normalized", *shape, seed=5, boot="row")
+    before = _one_launches()
+    _call(to_device(inp, device), params, columns=True)
+    assert _one_launches() - before == want
