@@ -162,7 +162,14 @@ std::map<std::pair<int, uintptr_t>, uint64_t>& workspace_calls() {
   return *m;
 }
 uint64_t g_ws_max_calls = RLK_WORKSPACE_MAX_CALLS;
-uint64_t g_ws_clears = 0;
+uint64_t g_ws_clears = 0, g_sync_clears = 0;  // (of workspaces; of normalised GAE's buffers)
+
+// A zero-filled byte buffer that is an ordinary tensor whatever mode the call runs in: one made
+// under inference mode could not be zero-filled again outside it.
+at::Tensor zeroed(int64_t bytes, const at::Tensor& like) {
+  const c10::InferenceMode ordinary(false);
+  return at::zeros({bytes}, like.options().dtype(at::kByte));
+}
 
 struct Workspace {
   void* ptr = nullptr;
@@ -187,7 +194,7 @@ Workspace workspace(const Call& c, const at::Tensor& like) {
   if (!buf.defined() || (size_t)buf.numel() < need) {
     size_t size = buf.defined() ? std::max(need, 2 * (size_t)buf.numel()) : need;
     size = (size + 255) / 256 * 256;
-    buf = at::zeros({(int64_t)size}, like.options().dtype(at::kByte));
+    buf = zeroed((int64_t)size, like);
     calls = 0;
   }
   if (calls >= g_ws_max_calls) {
@@ -226,9 +233,10 @@ bool ask_one_launch(const Call& c, const at::Tensor& like, rlk_time_major_call& 
   hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
   if (hipStreamIsCapturing(s, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone) return false;
   NormSync& n = norm_syncs()[{(int)c.dev, reinterpret_cast<uintptr_t>(s)}];
-  if (!n.buf.defined()) n.buf = at::zeros({(int64_t)RLK_NORM_SYNC_BYTES}, like.options().dtype(at::kByte));
+  if (!n.buf.defined()) n.buf = zeroed(RLK_NORM_SYNC_BYTES, like);
   if (n.epoch >= std::min<uint64_t>(g_ws_max_calls, RLK_NORM_MAX_EPOCH)) {
     n.buf.zero_();
+    ++g_sync_clears;
     n.epoch = 0;
   }
   t.sync = n.buf.data_ptr();
@@ -891,6 +899,7 @@ PyObject* norm_syncs_list(PyObject*, PyObject*) {
 PyObject* one_launches(PyObject*, PyObject*) { return PyLong_FromUnsignedLongLong(g_one_launches); }
 
 PyObject* workspace_clears(PyObject*, PyObject*) { return PyLong_FromUnsignedLongLong(g_ws_clears); }
+PyObject* sync_clears(PyObject*, PyObject*) { return PyLong_FromUnsignedLongLong(g_sync_clears); }
 
 PyMethodDef kMethods[] = {
     {"entry", make_entry, METH_VARARGS, "entry(op, names, npos, defaults, required, fallback)"},
@@ -899,6 +908,8 @@ PyMethodDef kMethods[] = {
      "cached workspace (n <= 0: the default, RLK_WORKSPACE_MAX_CALLS)"},
     {"workspace_clears", workspace_clears, METH_NOARGS,
      "workspace_clears() -> cached workspaces zero-filled again at the call limit so far"},
+    {"sync_clears", sync_clears, METH_NOARGS,
+     "sync_clears() -> buffers of normalised GAE in one launch zero-filled again at the call limit so far"},
     {"norm_syncs", norm_syncs_list, METH_NOARGS,
      "norm_syncs() -> [(device, epoch, buffer)] of normalised GAE calls in one launch"},
     {"one_launches", one_launches, METH_NOARGS,

@@ -231,7 +231,8 @@ def _workspace(dev: int, stream: int, n_env: int, n_t: int):
         cur = torch.cuda.current_stream(dev)
         if cur.cuda_stream != stream:
             raise RuntimeError("workspace stream mismatch")
-        ws = torch.zeros(size, dtype=torch.uint8, device=torch.device("cuda", dev))
+        with torch.inference_mode(False):  # an ordinary tensor: zero-filled again in any mode
+            ws = torch.zeros(size, dtype=torch.uint8, device=torch.device("cuda", dev))
         _workspaces[(dev, stream)] = ws
         _ws_calls[(dev, stream)] = 0
     _count_call((dev, stream), ws)

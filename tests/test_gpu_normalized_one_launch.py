@@ -82,6 +82,7 @@ def test_streams_and_call_limit(device, monkeypatch):
     d = to_device(inp, device)
     want = _two_launches(d, params)
     prev = _native.fast.set_workspace_max_calls(3)
+    clears = _native.fast.sync_clears()
     try:
         streams = [torch.cuda.Stream() for _ in range(2)]
         torch.cuda.synchronize()
@@ -91,6 +92,8 @@ def test_streams_and_call_limit(device, monkeypatch):
                 with torch.cuda.stream(s):
                     outs.append(_call(d, params))
         torch.cuda.synchronize()
+        # ten calls on each stream, at most three between two clears
+        assert _native.fast.sync_clears() - clears >= 2 * 3
         for out in outs:
             for g, w in zip(out, want):
                 assert torch.equal(g, w)
