@@ -53,6 +53,9 @@ typedef struct rlk_time_major_call {
  * actions up to 512 steps or at least 1024 environments.  Other calls are faster through
  * contiguous copies. */
 int rlk_time_major_takes(int64_t num_envs, int64_t seq_len, int64_t step_stride, int64_t num_actions);
+/* 1 if a taken call is also faster on the device than copying its `arrays` [num_envs, seq_len] arrays
+ * to rows, without the host's launches: what counts while a graph is captured. */
+int rlk_time_major_beats_copies(int op, int arrays, int64_t num_envs, int64_t seq_len, int64_t num_actions);
 size_t rlk_time_major_partials_bytes(int64_t num_envs, int64_t seq_len);
 int rlk_time_major(const rlk_time_major_call *call, void *stream);
 

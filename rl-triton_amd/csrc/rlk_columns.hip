@@ -46,6 +46,26 @@ bool takes(int64_t num_envs, int64_t T, int64_t ld, int64_t num_actions) {
          (num_envs + kCols - 1) / kCols <= kMaxLaunchBlocks && (num_actions <= 4 || T <= 512 || num_envs >= 1024);
 }
 
+// Whether the kernel takes less time on the device than a copy of each of the call's `arrays`
+// [E, T] arrays and the row kernel.  A call made eagerly waits for the host's launches first, and
+// one launch is faster at every shape taken (few environments, 2048 steps: prefix sum 16.7 us
+// against 20.0, GAE 20 against 40, Retrace 36 against 61); in a graph the device's time is all.
+// A pass over 256 steps costs about a copy of a small array, 2 us (quarters of it by op below),
+// whatever the environments until they fill the GPU; copies grow with the elements.  Replayed from
+// a graph on MI355X, copies against this, us: prefix sum [16,512] 7.1, 5.7, [16,1024] 7.3, 9.3,
+// [64,2048] 8.1, 17.0, [512,2048] 19.2, 17.5; GAE with truncations [16,1280] 14.4, 13.7, [16,2048]
+// 14.2, 19.9, [128,2048] 21.3, 20.1; V-trace [16,2048] 14.5, 23.1, [256,2048] 27.5, 23.6; Retrace
+// A = 4 [16,1536] 23.6, 28.3, [64,1536] 30.5, 27.3; normalised GAE [64,2048] 13.6, 25.5.  Of 800
+// calls of 2 to 2000 environments the rule is wrong by more than 10% at four (V-trace with
+// truncations [64,2048] 21.1, 25.6; masked GAE [2,1024] 10.6, 12.4).
+bool beats_copies(int op, int arrays, int64_t num_envs, int64_t T, int64_t num_actions) {
+  if (op == RLK_OP_RETRACE && num_actions > 4) return true;  // (takes has a rule of its own)
+  const int64_t passes = (T + 255) / 256;
+  const int quarters = op == RLK_OP_RETRACE ? 7 : op == RLK_OP_GAE_NORMALIZED ? 6
+                       : op == RLK_OP_GAE || op == RLK_OP_VTRACE ? 5 : 4;
+  return quarters * passes <= 4 * (arrays + 1) + 4 * arrays * num_envs * T / 350000;
+}
+
 template <class E>
 const E* in_of(const rlk_time_major_call& c, int i) { return static_cast<const E*>(c.in[i]); }
 template <class E>
@@ -147,6 +167,10 @@ extern "C" {
 
 int rlk_time_major_takes(int64_t num_envs, int64_t seq_len, int64_t step_stride, int64_t num_actions) {
   return takes(num_envs, seq_len, step_stride, num_actions) ? 1 : 0;
+}
+
+int rlk_time_major_beats_copies(int op, int arrays, int64_t num_envs, int64_t seq_len, int64_t num_actions) {
+  return beats_copies(op, arrays, num_envs, seq_len, num_actions) ? 1 : 0;
 }
 
 int rlk_time_major_one_launch_takes(int64_t num_envs, int64_t seq_len) {

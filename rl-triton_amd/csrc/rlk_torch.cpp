@@ -140,6 +140,18 @@ rlk_time_major_call time_major(const Call& c, int op, const at::Tensor* const* t
   return t;
 }
 
+// A time-major call being captured into a graph that is faster there as copies and a row kernel
+// (the Python path's): to be declined.
+bool copied_in_graph(const Call& c, const rlk_time_major_call& t) {
+  if (c.T <= 512) return false;  // (one or two passes never lose)
+  int arrays = t.boot_mode == RLK_BOOT_FULL ? 1 : 0;
+  for (const void* p : t.in) arrays += p != nullptr;
+  if (rlk_time_major_beats_copies(t.op, arrays, c.E, c.T, t.num_actions)) return false;
+  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+  return hipStreamIsCapturing(static_cast<hipStream_t>(c.stream()), &cs) == hipSuccess &&
+         cs != hipStreamCaptureStatusNone;
+}
+
 // Look-back workspaces of the calls this module launches, one per (device, stream):
 // zero-filled when allocated (on that stream), grown by doubling, and left ready by every
 // call for the next.  Calls on one stream are ordered, so one buffer serves them all, and
@@ -345,6 +357,7 @@ PyObject* op_gae(PyObject* const* a, Py_ssize_t n) {
   if (c.ld > 0) {
     const at::Tensor* in[] = {r, v, te, tr, mask};
     rlk_time_major_call t = time_major(c, RLK_OP_GAE, in, 5, boot, mode);
+    if (copied_in_graph(c, t)) return decline();
     t.gamma = gamma, t.lambda_ = lam;
     at::Tensor out = c.output(*r);
     t.out[0] = out.data_ptr();
@@ -389,6 +402,7 @@ PyObject* op_gae_normalized(PyObject* const* a, Py_ssize_t n) {
   if (c.ld > 0) {
     const at::Tensor* in[] = {r, v, te, tr, mask};
     rlk_time_major_call t = time_major(c, RLK_OP_GAE_NORMALIZED, in, 5, boot, mode);
+    if (copied_in_graph(c, t)) return decline();
     t.gamma = gamma, t.lambda_ = lam, t.eps = eps;
     at::Tensor adv = c.output(*r), ret = c.output(*r);
     if (one_launch_shape(c, mask != nullptr) && ask_one_launch(c, *r, t)) {
@@ -461,6 +475,7 @@ PyObject* op_vtrace(PyObject* const* a, Py_ssize_t n) {
   if (c.ld > 0) {
     const at::Tensor* in[] = {lpt, lpb, v, r, te, tr};
     rlk_time_major_call t = time_major(c, RLK_OP_VTRACE, in, 6, boot, mode);
+    if (copied_in_graph(c, t)) return decline();
     t.gamma = gamma, t.rho_bar = rho_bar, t.c_bar = c_bar;
     at::Tensor tg = c.output(*r), adv = c.output(*r);
     t.out[0] = tg.data_ptr(), t.out[1] = adv.data_ptr();
@@ -509,6 +524,7 @@ PyObject* op_retrace(PyObject* const* a, Py_ssize_t n) {
     const at::Tensor* in[] = {pi, mu, q, nq, act, r, te, tr};
     rlk_time_major_call t = time_major(c, RLK_OP_RETRACE, in, 8, nullptr, RLK_BOOT_NONE);
     t.num_actions = A, t.gamma = gamma, t.lambda_ = lam, t.rho_bar = rho_bar, t.c_bar = c_bar;
+    if (copied_in_graph(c, t)) return decline();
     at::Tensor tg = c.output(*r), adv = c.output(*r);
     t.out[0] = tg.data_ptr(), t.out[1] = adv.data_ptr();
     return finish(rlk_time_major(&t, c.stream()), "rlk_time_major", pair(tg, adv));
@@ -544,6 +560,7 @@ PyObject* op_lambda_returns(PyObject* const* a, Py_ssize_t n) {
   if (c.ld > 0) {
     const at::Tensor* in[] = {r, nv, te, tr};
     rlk_time_major_call t = time_major(c, RLK_OP_LAMBDA_RETURNS, in, 4, boot, boot ? RLK_BOOT_FULL : RLK_BOOT_NONE);
+    if (copied_in_graph(c, t)) return decline();
     t.gamma = gamma, t.lambda_ = lam;
     at::Tensor out = c.output(*r);
     t.out[0] = out.data_ptr();
@@ -578,6 +595,7 @@ PyObject* op_discounted_returns(PyObject* const* a, Py_ssize_t n) {
   if (c.ld > 0) {
     const at::Tensor* in[] = {r, te, tr};
     rlk_time_major_call t = time_major(c, RLK_OP_DISCOUNTED_RETURNS, in, 3, boot, boot ? RLK_BOOT_FULL : RLK_BOOT_NONE);
+    if (copied_in_graph(c, t)) return decline();
     t.gamma = gamma;
     at::Tensor out = c.output(*r);
     t.out[0] = out.data_ptr();
@@ -611,6 +629,7 @@ PyObject* op_eligibility_traces(PyObject* const* a, Py_ssize_t n) {
   if (c.ld > 0) {
     const at::Tensor* in[] = {g, d};
     rlk_time_major_call t = time_major(c, RLK_OP_FORWARD, in, 2, seed, RLK_BOOT_NONE);
+    if (copied_in_graph(c, t)) return decline();
     t.gamma = gamma * lam, t.ends_at = 1;
     at::Tensor out = c.output(*g);
     t.out[0] = out.data_ptr();
@@ -642,6 +661,7 @@ PyObject* op_prefix_sum(PyObject* const* a, Py_ssize_t n) {
   if (c.ld > 0) {
     const at::Tensor* in[] = {x, d};
     rlk_time_major_call t = time_major(c, RLK_OP_FORWARD, in, 2, seed, RLK_BOOT_NONE);
+    if (copied_in_graph(c, t)) return decline();
     t.gamma = 1.f, t.ends_at = a[3] == Py_True ? 1 : 0;
     at::Tensor out = c.output(*x);
     t.out[0] = out.data_ptr();

@@ -280,3 +280,25 @@ def test_noalloc_entry_refuses_before_any_device_call():
     assert lib.rlk_gae_noalloc(None, None, None, None, None, 0, None, 0, 5000, 0.99, 0.95, None) == 0
     assert b"static buffer" in lib.rlk_status_string(-4)
     assert b"device" in lib.rlk_status_string(-5)
+
+
+def test_time_major_calls_against_copies():
+    """rlk_time_major_beats_copies: passes of 256 steps against copies of the call's arrays; never
+    worse with more environments, with more arrays or with fewer steps."""
+    f = ctypes.CDLL(_native.library_path()).rlk_time_major_beats_copies
+    f.argtypes = [ctypes.c_int, ctypes.c_int, ctypes.c_int64, ctypes.c_int64, ctypes.c_int64]
+    gae, normalized, vtrace, retrace, lam, disc, fwd = range(7)
+    # (op, arrays, environments, steps, actions) as measured
+    for call, want in [((fwd, 2, 16, 512, 0), 1), ((fwd, 2, 16, 1024, 0), 0), ((fwd, 2, 512, 2048, 0), 1),
+                       ((gae, 5, 16, 1280, 0), 1), ((gae, 5, 16, 2048, 0), 0), ((gae, 5, 128, 2048, 0), 1),
+                       ((vtrace, 5, 64, 2048, 0), 0), ((vtrace, 5, 256, 2048, 0), 1), ((retrace, 8, 16, 1536, 4), 0),
+                       ((retrace, 8, 64, 1536, 4), 1), ((normalized, 3, 64, 2048, 0), 0), ((disc, 2, 256, 1024, 0), 1),
+                       ((lam, 5, 16, 1536, 0), 1), ((lam, 5, 16, 2048, 0), 0), ((retrace, 8, 1024, 2048, 18), 1)]:
+        assert f(*call) == want, call
+    for op, few, many in ((gae, 3, 6), (normalized, 3, 6), (vtrace, 5, 7), (retrace, 7, 8), (lam, 3, 5), (disc, 2, 4),
+                          (fwd, 2, 2)):
+        for arrays in range(few, many + 1):
+            takes = [[f(op, arrays, e, t, 0) for t in range(16, 2049, 16)] for e in (1, 16, 100, 400, 2000, 100000)]
+            assert all(row[:32] == [1] * 32 for row in takes), "up to 512 steps: always"
+            for fewer, more in zip(takes, takes[1:]):
+                assert all(a <= b for a, b in zip(fewer, more))

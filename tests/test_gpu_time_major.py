@@ -192,3 +192,39 @@ def test_time_major_order_of_streams(device, no_flags):
             x.fill_(float(i))
             got = rl_triton.compute_episodic_prefix_sum(x.t(), torch.zeros_like(x).t())
             assert torch.equal(got[:, -1], torch.full((256,), 128.0 * i, device=device))
+
+
+@pytest.mark.parametrize("op,boot,shape,copied", [
+    ("prefix_sum", "none", (16, 512), False), ("prefix_sum", "none", (16, 1024), True),
+    ("prefix_sum", "none", (600, 2048), False), ("gae", "full", (16, 1024), False), ("gae", "full", (16, 2048), True),
+    ("vtrace", "row", (64, 2048), True), ("retrace", "none", (16, 1024), False), ("retrace", "none", (16, 2048), True),
+    ("gae_normalized_masked", "row", (64, 2048), True), ("discounted_returns", "none", (64, 2048), True)],
+    ids=lambda v: f"{v[0]}x{v[1]}" if isinstance(v, tuple) else None)
+def test_captured_calls_take_the_faster_form(op, boot, shape, copied, device, no_flags):
+    """In a graph the device's time is all that counts: calls of few environments and many steps are
+    captured as copies and the row kernel (the bits of the call on contiguous arrays), others as the
+    time-major kernel (the bits of the eager call).  Eager calls take the kernel."""
+    from rl_triton import _native
+    inp, params = _inputs(op, shape, boot, 0.02 if boot == "full" else 0.0)
+    d = _columns(inp, device)
+    rows = {k: None if v is None else v.contiguous() for k, v in d.items()}
+    before = _native.fast.launched()
+    want = [t.clone() for t in _call(op, d, params)]
+    assert _native.fast.launched() == before + 1
+    if copied:
+        # two launches of a normalised call have the bits of its one launch
+        want = [t.clone() for t in _call(op, rows, params)]
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    before = _native.fast.launched()
+    with torch.cuda.graph(graph):
+        got = _call(op, d, params)
+    assert _native.fast.launched() - before == (0 if copied else 1)
+    for _ in range(3):
+        for t in got:
+            t.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        for g, w in zip(got, want):
+            assert torch.equal(g, w)
+    del graph
