@@ -290,7 +290,7 @@ def test_time_major_calls_against_copies():
     gae, normalized, vtrace, retrace, lam, disc, fwd = range(7)
     # (op, arrays, environments, steps, actions) as measured
     for call, want in [((fwd, 2, 16, 512, 0), 1), ((fwd, 2, 16, 1024, 0), 0), ((fwd, 2, 512, 2048, 0), 1),
-                       ((gae, 5, 16, 1280, 0), 1), ((gae, 5, 16, 2048, 0), 0), ((gae, 5, 128, 2048, 0), 1),
+                       ((gae, 5, 16, 1280, 0), 1), ((gae, 5, 16, 2048, 0), 0), ((gae, 5, 256, 2048, 0), 1),
                        ((vtrace, 5, 64, 2048, 0), 0), ((vtrace, 5, 256, 2048, 0), 1), ((retrace, 8, 16, 1536, 4), 0),
                        ((retrace, 8, 64, 1536, 4), 1), ((normalized, 3, 64, 2048, 0), 0), ((disc, 2, 256, 1024, 0), 1),
                        ((lam, 5, 16, 1536, 0), 1), ((lam, 5, 16, 2048, 0), 0), ((retrace, 8, 1024, 2048, 18), 1)]:
