@@ -1,5 +1,6 @@
-"""The look-back path (rows longer than 2048 steps) in the layouts the BASELINE shapes do not
-reach: more rows than counter slots (64), so that several rows share a slot; rows of many
+"""The look-back path (rows of more than 16384 steps; from 2049 or 8193 steps on where a workgroup
+does not hold the row whole, whole_row_segments in csrc/rlk_launch.hpp) in the layouts the BASELINE
+shapes do not reach: more rows than counter slots (64), so that several rows share a slot; rows of many
 tiles; one workspace serving calls of changing shapes in stream order; two streams at once;
 the rare paths (a predecessor computed in its workgroup's place, a walk back past 64 tiles,
 a wait that gives up) forced from the host; and every op at those shapes.  Against the float64 oracle with the long-row
@@ -55,9 +56,11 @@ def _check(op, E, T, seed, device):
 
 
 @pytest.mark.parametrize("op", OPS)
-@pytest.mark.parametrize("shape", [(65, 2049), (130, 4100), (200, 2052)],
+@pytest.mark.parametrize("shape", [(65, 2049), (130, 4100), (200, 2052), (65, 9001), (100, 8200), (70, 16400)],
                          ids=lambda s: f"{s[0]}x{s[1]}")
 def test_more_rows_than_slots(op, shape, device):
+    """(The first three shapes are tiles for Retrace with 130 rows of 4100 steps only, and otherwise
+    rows held whole.)"""
     from rl_triton import _native
     _check(op, *shape, seed=21, device=device)
     assert not _native.workspace_error(device)
@@ -144,13 +147,17 @@ def test_single_tile_rows_between_chained_calls(path, device, monkeypatch):
     """Calls of one tile per row skip the look-back protocol and leave the workspace as
     they found it.  On a new stream (a new, zeroed workspace), such calls queued between
     chained ones, of changing row counts: every chained call must still find its slots'
-    epochs current and its counters at rest.  Every result matches the oracle and no wait
-    gives up."""
+    epochs current and its counters at rest.  (Such rows have 8193 to 16384 steps, and 13001 pads a
+    16384-step tile least; shorter ones are held whole and do not touch the workspace either.)
+    Every result matches the oracle and no wait gives up."""
     import torch
     from rl_triton import _native
     if path == "fast":
         monkeypatch.delenv("RL_TRITON_CORRECTNESS_WARNINGS")
-    shapes = [("prefix_sum", 300, 3000), ("prefix_sum", 2, 300000), ("discounted_returns", 1000, 2101),
+    shapes = [("prefix_sum", 70, 12801), ("prefix_sum", 5, 90000), ("discounted_returns", 100, 13001),
+              ("discounted_returns", 70, 20001), ("gae", 100, 13000), ("gae", 65, 9001),
+              ("eligibility_traces", 5, 12291), ("lambda_returns", 64, 13001), ("lambda_returns", 2, 150000),
+              ("prefix_sum", 300, 3000), ("prefix_sum", 2, 300000), ("discounted_returns", 1000, 2101),
               ("discounted_returns", 3, 200001), ("gae", 70, 4000), ("prefix_sum", 70, 9000),
               ("eligibility_traces", 512, 2500), ("prefix_sum", 1, 600000), ("vtrace", 100, 4096),
               ("vtrace", 2, 131073)]
@@ -220,35 +227,6 @@ def test_lookback_give_up_poisons_with_nan(device):
     assert_close(g[~nan], exp[~nan], 1e-5, _atol(op, inp, exp), f"{op}[{E},{T}] outside the NaN tiles")
 
 
-@pytest.mark.parametrize("path", ["python", "fast"])
-def test_single_tile_rows_between_chained_calls(path, device, monkeypatch):
-    """Calls of one tile per row skip the look-back protocol and leave the workspace as
-    they found it.  On a new stream (a new, zeroed workspace), such calls queued between
-    chained ones, of changing row counts: every chained call must still find its slots'
-    epochs current and its counters at rest.  Every result matches the oracle and no wait
-    gives up."""
-    import torch
-    from rl_triton import _native
-    if path == "fast":
-        monkeypatch.delenv("RL_TRITON_CORRECTNESS_WARNINGS")
-    shapes = [("prefix_sum", 300, 3000), ("prefix_sum", 2, 300000), ("discounted_returns", 1000, 2101),
-              ("discounted_returns", 3, 200001), ("gae", 70, 4000), ("prefix_sum", 70, 9000),
-              ("eligibility_traces", 512, 2500), ("prefix_sum", 1, 600000), ("vtrace", 100, 4096),
-              ("vtrace", 2, 131073)]
-    stream = torch.cuda.Stream(device)
-    pending = []
-    with torch.cuda.stream(stream):
-        for i, (op, E, T) in enumerate(shapes * 2):
-            inp, params = _inputs(op, E, T, seed=700 + i)
-            pending.append((op, E, T, inp, params, run_api(op, inp, params, device)))
-    torch.cuda.synchronize()
-    for op, E, T, inp, params, got in pending:
-        exp = run_oracle(op, inp, params)
-        for name, g, e in zip(OUTPUTS[op], got, exp):
-            assert_close(g.cpu().numpy(), e, 1e-5, _atol(op, inp, e), f"{op}[{E},{T}] in sequence:{name}")
-    assert not _native.workspace_error(device)
-
-
 @pytest.mark.parametrize("op,shape", [("prefix_sum", (1, 1 << 23)), ("vtrace", (1, 1 << 21)),
                                       ("gae_masked", (2, 1 << 19)), ("retrace", (3, 70000)),
                                       ("discounted_returns", (16, 131072)),
@@ -293,9 +271,8 @@ def test_tiles_between_one_and_two_per_cu(op, shape, device):
     ops whose tiles can double take 16384-step tiles, fewer than the CUs, in one round;
     V-trace, whose largest tile is 8192 steps, takes 512 x 2 so that two workgroups fit a
     CU.  Aligned and element-aligned rows, with truncations where the op has them, and
-    bfloat16 bit-identical to the float32 result rounded.  On a 256-CU MI355X, 257 and 512
-    tiles ([257,8192], [256,16384]) are the rules' edges and 513 and 256 ([171,24576],
-    [256,8192]) fall just outside them."""
+    bfloat16 bit-identical to the float32 result rounded.  ([257,8192], [256,8192] and
+    [256,16384] are held whole; so is [200,10001] but for GAE and V-trace.)"""
     import torch
     from rl_triton import _native
     _check(op, *shape, seed=61, device=device)
@@ -315,9 +292,10 @@ def test_tiles_between_one_and_two_per_cu(op, shape, device):
                          ids=lambda s: f"{s[0]}x{s[1]}")
 def test_rows_much_shorter_than_the_cu_tile(op, shape, device):
     """Many rows of a few thousand steps, where the tile that gives every CU one would be
-    mostly padding: the launcher takes smaller tiles (4096 steps at 512 threads, or the
-    op's 8192-step ones), one to three per row with a ragged last tile, aligned and
-    element-aligned rows.  And few rows whose smallest CU-sized tiles leave CUs idle
+    mostly padding: most are held whole by a workgroup each; the others (Retrace,
+    element-aligned GAE and V-trace [300,10001], [64,12000]) take smaller tiles (4096 steps
+    at 512 threads, or the op's 8192-step ones), one to three per row with a ragged last
+    tile, aligned and element-aligned rows.  And few rows whose smallest CU-sized tiles leave CUs idle
     ([16,40000], [24,20001]): 4096-step tiles, five to ten per row.  Against the oracle,
     and bfloat16 bit-identical to the float32 result rounded."""
     import torch
@@ -363,12 +341,14 @@ def test_discounted_returns_wide_tiles(shape, boot, device):
 
 
 @pytest.mark.parametrize("op,shape", [("vtrace", (2048, 16384)), ("prefix_sum", (1024, 1 << 16)),
-                                      ("gae_masked", (600, 12000))],
+                                      ("gae_masked", (600, 12000)), ("vtrace", (700, 20000)),
+                                      ("gae_masked", (400, 20001)), ("gae", (300, 15001))],
                          ids=lambda v: v if isinstance(v, str) else f"{v[0]}x{v[1]}")
 def test_grids_larger_than_the_gpu(op, shape, device):
     """Thousands of multi-tile rows: far more workgroups than the GPU holds at once, so tiles
     wait on predecessors that may not have started; every result matches the oracle and no
-    wait gives up."""
+    wait gives up.  (V-trace [2048,16384] and masked GAE [600,12000] are held whole, a workgroup
+    per row; GAE [300,15001] is one tile per row.)"""
     from rl_triton import _native
     _check(op, *shape, seed=73, device=device)
     assert not _native.workspace_error(device)

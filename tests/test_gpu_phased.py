@@ -12,7 +12,8 @@ sit at another phase than its inputs takes the element-aligned path instead; bot
 the oracle.  A row's tiles are shifted to its four-element boundaries, which leaves up to
 3 steps of the row outside them (backward scans: at the row's end, forward: at its start);
 the first tile in scan order takes those as one more quad.  Lengths just below a multiple
-of the tile (8190, 12287, 131071, 262143) put them beyond the last tile.
+of the tile (12287, 16381, 131071, 262143) put them beyond the last tile.  (Rows of 4097 to 8190
+steps here are held whole by a workgroup and take element-aligned access.)
 """
 import numpy as np
 import pytest
@@ -26,7 +27,7 @@ CASES = [("gae", 5, 8190), ("gae_masked", 5, 4099), ("vtrace", 3, 12287),
          ("lambda_returns", 7, 4097), ("discounted_returns", 4, 65539),
          ("discounted_returns", 16, 131071), ("eligibility_traces", 6, 8193),
          ("prefix_sum", 8, 20001), ("prefix_sum", 3, 262143), ("backward_scan", 3, 16383),
-         ("forward_scan", 9, 9001)]
+         ("forward_scan", 9, 9001), ("gae", 5, 16381), ("gae_masked", 5, 12291), ("lambda_returns", 7, 8197)]
 
 
 def _inputs(op, E, T, seed):

@@ -12,8 +12,9 @@ must equal the result for the pattern; the split falls inside a repetition.
 * Every other op at [4096 * 65537, 3] (split alike), its arrays advanced by whole rows in
   each launch: [E, T], [E, T, A] (Retrace) and per-row ones (bootstrap, seed), against the
   float64 oracle on the pattern.
-* Long rows, [4096 * 1025, 2049] in bfloat16 (one 32768-step tile per row, 4198400
-  workgroups of 1024 threads, split 4193792 + 4608 rows; T odd, so phased access): the
+* Long rows in bfloat16: [4096 * 1025, 2049] (a workgroup per row, 4198400 of them, split
+  4193792 + 4608 rows) and [4096 * 205, 16401] (five 4096-step tiles per row, as many workgroups,
+  split 838656 + 1024 rows; T odd, so phased access): the
   episodic prefix sum with seeds, bit-identical in every repetition to the float32
   kernels' result for the pattern rounded (rows at the same element placement), which is
   itself checked against the float64 oracle.
@@ -96,10 +97,10 @@ def test_normalized_gae_short_rows_over_two_launches(device, big_memory):
     assert _worst(adv, adv_exp, k, 1e-5, 2e-5) <= 0.0
 
 
-def test_prefix_sum_long_rows_over_two_launches_bf16(device, big_memory):
+@pytest.mark.parametrize("k,T,gib", [(1025, 2049, 64), (205, 16401, 96)], ids=["whole", "tiles"])
+def test_prefix_sum_long_rows_over_two_launches_bf16(k, T, gib, device, big_memory):
     import rl_triton
-    k, T = 1025, 2049
-    big_memory(64)
+    big_memory(gib)
     print(f"[split] prefix_sum bf16 [{P * k},{T}]", flush=True)
     pat, params = make_inputs("prefix_sum", P, T, seed=3, boot="row", p_done=1e-3)
     pat = {n: torch.as_tensor(v).to(torch.bfloat16).float().numpy() for n, v in pat.items()

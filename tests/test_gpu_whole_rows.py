@@ -16,12 +16,12 @@ OPS = ["gae", "gae_masked", "gae_normalized", "gae_normalized_masked", "vtrace",
 # four-segment ones with a row for half the CUs of a 256-CU GPU, and one row fewer
 @pytest.mark.parametrize("shape", [(3, 2049), (2, 2052), (5, 2304), (2, 2305), (3, 4095), (2, 4096), (3, 4097),
                                    (2, 4100), (300, 4609), (257, 8191), (2, 8192), (127, 8193), (128, 8193),
-                                   (129, 8196), (130, 9217), (128, 16383), (128, 16384)],
+                                   (129, 8196), (130, 9217), (128, 9002), (128, 16383), (128, 16384)],
                          ids=lambda s: f"{s[0]}x{s[1]}")
 @pytest.mark.parametrize("op", OPS)
 def test_whole_rows(op, shape, device):
-    if op in ("prefix_sum", "gae_masked", "gae_normalized_masked") and shape[0] * shape[1] > 1 << 20 and shape[1] % 4:
-        pytest.skip("the aligned neighbours cover these in full size")
+    if op in ("prefix_sum", "gae_masked", "gae_normalized_masked") and shape[0] * shape[1] > 1 << 21 and shape[1] % 4:
+        pytest.skip("the oracle is slow here; the smaller element-aligned shapes cover each segment count")
     kw = {"p_done": 1e-2} if op in ("prefix_sum", "eligibility_traces") else {}
     trunc = 0.01 if op in ("gae", "vtrace", "gae_normalized") else 0.0
     inp, params = make_inputs(op, *shape, seed=shape[0] + shape[1], p_trunc=trunc,
