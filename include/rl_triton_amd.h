@@ -104,7 +104,10 @@ size_t rlk_workspace_bytes(int64_t num_envs, int64_t seq_len);
  * a state walks further back (fallback_polls; default 256).  Negative values restore the
  * defaults.  A wait that gives up sets the workspace error flag and writes NaN for its
  * tile and every tile that chains through it; with the defaults a correct run never gets
- * there.  The fallback paths give the same bits as the ordinary one.  Returns RLK_OK. */
+ * there.  fallback_polls is also how often a workgroup of a normalised GAE in one launch
+ * (rlk_time_major.h) looks for the others' statistics before it leaves raw advantages for
+ * them to normalise.  The fallback paths give the same bits as the ordinary one.  Returns
+ * RLK_OK. */
 int rlk_debug_lookback(int give_up_polls, int fallback_polls);
 
 /* For tests of the output stores only; no counterpart in the reference.  The kernels store

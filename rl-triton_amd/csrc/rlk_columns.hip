@@ -39,8 +39,11 @@ int launch_columns(const Op& op, const rlk_time_major_call& c, hipStream_t strea
 
 // Rows above 2048 steps are few and are split over workgroups, which the row kernels do.  Retrace
 // with any action count waits for its action rows in every pass of 128 steps (8.7 us at A = 18):
-// more than four passes of few environments lose to copying the arrays to rows ([64,1000] 70
-// against 55 us per call, [1000,500] 41 against 211).
+// more than four passes of few environments lose to copying the arrays to rows.  Per call, copies
+// against this, us: A = 18 [64,1000] 63, 69, [64,2048] 61, 141, [256,2048] 80, 142; A = 6 [64,2048]
+// 64, 93; and [1000,500] 211, 41, [1000,1000] 171, 74.  (The line is on the copies' side of the
+// crossover: calls that this would serve faster lie beyond it, A = 18 [64,600] 61, 43, A = 6
+// [64,1000] 61, 44.)
 bool takes(int64_t num_envs, int64_t T, int64_t ld, int64_t num_actions) {
   return num_envs > 0 && T > 0 && T <= kShortMaxT && ld >= num_envs &&
          (num_envs + kCols - 1) / kCols <= kMaxLaunchBlocks && (num_actions <= 4 || T <= 512 || num_envs >= 1024);

@@ -834,8 +834,14 @@ __global__ __launch_bounds__(NT) void normalize_kernel(E* __restrict__ x,
 //
 // Bound by the trips of the statistics through memory between the XCDs.  Calls in a row, us per
 // call, two launches -> one: [64,64] 9.4 -> 4.7, [1024,128] 9.2 -> 4.9, [4096,128] 9.2 -> 7.5 (all
-// paced by the host before; on the device 7.1 -> 7.3), [256,4096] 11.4 -> 9.0, [256,8192]
-// 17.3 -> 11.6, [200,12000] 18.5 -> 12.1.
+// paced by the host before; where the device sets the pace, 256 workgroups of short rows are 2%
+// slower in one launch: [4096,128] 8.1 -> 8.3, masked 8.6 -> 8.8), [256,4096] 11.4 -> 9.0,
+// [256,8192] 17.3 -> 11.6, [200,12000] 18.5 -> 12.1.
+// Beside other work on the GPU resident workgroups hold their CUs while they wait for room for the
+// rest, up to `polls` reads (350 us).  Next to matrix products or copies on another stream one
+// launch was no slower than two all the same: [64,64] 9.5 -> 7.2 us beside copies, [256,2048]
+// 57 -> 58 beside 4096^3 products, [512,6000] masked 77 -> 68; the other stream lost up to 3%
+// (0.5 GB copies beside [512,6000], 232 -> 238 us each).
 constexpr int kNormWords = 4;  // three doubles in 4 x 48 bits
 constexpr int kNormPollers = 256;  // threads that poll, for one or two workgroups each
 constexpr int kNormMaxBlocks = 2 * kNormPollers;

@@ -268,10 +268,13 @@ bool step_per_thread(int64_t E, int64_t T) {
 }
 
 // Rows of more than 2048 steps that one workgroup holds whole (rows_strided_kernel, as many waves
-// as the row needs): no look-back, no padding to a tile, few enough registers that two or more
-// workgroups share a CU (Q segments of 4 steps per thread: up to 1024 * 4 * Q steps).  Against
-// the look-back's tiles, on MI355X (us):
-//   * up to 8192 steps (Q = 1, 2) faster at every count of rows: GAE [4,2500] by 1.46x, [64,2049]
+// as the row needs): no look-back, no padding to a tile, and for most ops up to 8192 steps few enough
+// registers that two or more workgroups share a CU (Q segments of 4 steps per thread: up to
+// 1024 * 4 * Q steps).  (The masked ops' Q = 2 instances hold 71 to 73 registers: two workgroups of
+// up to 12 waves; the statistics ops' masked Q = 4 ones 128, and spill up to 20 bytes per lane: one.)
+// Against the look-back's tiles, on MI355X (us):
+//   * up to 8192 steps (Q = 1, 2) faster at every count of rows, from one on (0.53-0.99 of the tiles' time
+//     for seven calls at 1 to 128 rows of 2049 to 8191 steps): GAE [4,2500] by 1.46x, [64,2049]
 //     4.34 -> 2.73, [512,5000] 12.2 -> 11.2, masked GAE [512,6000] 14.6 -> 10.6, [2000,5000]
 //     49.1 -> 34.1, V-trace [512,5000] 18.2 -> 13.3, bfloat16 [512,6000] 15.7 -> 9.3, TD(lambda)
 //     [2000,2049] 15.7 -> 11.1, prefix sum [2000,2049] 14.7 -> 9.2, [256,8192] 5.4 -> 4.6;

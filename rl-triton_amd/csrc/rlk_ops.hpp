@@ -413,12 +413,17 @@ struct VtraceOp {
 // rows start in different banks), and lane l sums row l in order of the actions, the order
 // (and the bits) of a loop over the row.  The next 64 rows' loads are issued before the sums.
 // Short rows go 128 or 256 at a time (bfloat16 A = 6 [1024,250] 6.7 us at 64 rows), rows of
-// more than kPipedActions actions in slices of 16 actions.
+// more than kPipedActions actions in slices of 16 actions.  (The cap is where the largest
+// straight-line batch that was built ends; 19 actions would fit the same LDS.  Slices cost a step
+// there, and another from 33 actions on, us: [1024,256] A = 17 8.9, 18 10.2, 19 14.4, 24 15.4,
+// 32 15.9, 33 20.0, 64 28.3; [4096,128] A = 17 15.0, 18 15.6, 19 19.4, 24 21.9.)
 //
 // Bound by HBM: on MI355X, float32, lane-by-lane rows -> this: A = 18 [4096,128] 78.3 -> 15.8
 // us (94 MB, 6.0 TB/s), [256,2048] 138.6 -> 16.8, [64,8192] 115.5 -> 23.8; A = 6 [4096,128]
 // 23.9 -> 8.6; bfloat16 A = 18 [4096,128] 108.1 -> 11.5.  A branch around each load or LDS
-// read instead of the straight-line batches took 28.4 us at A = 18 [4096,128].
+// read instead of the straight-line batches took 28.4 us at A = 18 [4096,128].  Lane-by-lane
+// rows were faster for bfloat16 A = 5 between 131072 and 262144 steps only ([1024,256] 5.2 us,
+// 5.4 so; [2000,100] 4.8, 5.5).
 //
 // LDS is the wave's own, dynamic (action_stage_bytes per wave): no barrier.
 // ------------------------------------------------------------------------------------------
@@ -429,8 +434,8 @@ __device__ __forceinline__ uint32_t load_word_ua(const float* p) { return __floa
 __device__ __forceinline__ uint32_t load_word_ua(const bf16* p) { return *reinterpret_cast<const ua_u1*>(p); }
 __host__ __device__ inline int action_stage_stride(int A) { return A <= kPipedActions ? (A | 1) : (kActionSlice | 1); }
 // Two staged arrays of 64 rows (rows of up to 9 actions: 128, up to 5: 256), the last row read
-// up to its batch's loads; later two result arrays of up to 256 steps.  At most 10 KB: sixteen
-// waves per CU.
+// up to its batch's loads; later two result arrays of up to 256 steps.  At most 9728 bytes (17 and
+// 18 actions): sixteen waves per CU.
 __host__ __device__ inline int action_stage_bytes(int A) {
   const int rows = kWave * (A <= 5 ? 4 : A <= 9 ? 2 : 1);
   const int batch = A <= 5 ? 5 : A <= 6 ? 6 : A <= 9 ? 9 : A <= 12 ? 12 : kPipedActions;
