@@ -10,6 +10,7 @@ namespace {
 // long-row tiles).
 size_t gae_normalized_partials(int64_t num_envs, int64_t seq_len) {
   if (num_envs <= 0 || seq_len <= 0) return 0;
+  const CusScope cus;
   const int64_t a = call_blocks<GaeStatsOp<true>>(num_envs, seq_len);
   const int64_t b = call_blocks<MaskedGaeStatsOp<true>>(num_envs, seq_len);
   return (size_t)partials_triples(a > b ? a : b) * kStatWords * sizeof(double);
@@ -23,6 +24,7 @@ int normalized_launch(StatsOp op, E* advantages, int64_t num_envs, int64_t seq_l
                       float eps, void* workspace, size_t workspace_bytes, void* partials,
                       size_t partials_bytes, void* stream) {
   if (num_envs < 0 || seq_len < 0 || seq_len > (int64_t{1} << 30)) return RLK_ERR_INVALID_ARGUMENT;
+  const CusScope cus;
   const int64_t nparts = call_blocks<StatsOp>(num_envs, seq_len);
   if (!partials_fit(partials, partials_bytes, nparts)) return RLK_ERR_WORKSPACE;
   op.partials = reinterpret_cast<double*>(partials);
